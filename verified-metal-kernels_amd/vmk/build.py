@@ -11,7 +11,11 @@ LIB = os.path.join(HERE, "libvmk.so")
 ARCH = "gfx950"
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
          # packed fp32 VALU forms are disabled: ordinary float code must not turn into them.
-         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+         "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         # MFMA accumulators in VGPRs.  A kernel whose LDS leaves one wave per SIMD may use 512 registers, and the
+         # compiler then keeps accumulators in AGPRs, which VALU code (the softmax rescale, the partial stores) reaches
+         # through copies only: 736 copies in the four-wave attention walks of one kernel, 64 and more per tile.
+         "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 
 
 def sources():
