@@ -1,0 +1,67 @@
+"""The two launches of the key split (decode and verification up to 64 rows per KV head): a call with few splits deals
+units of keys out to all waves and folds them in its combine launch, a call that fills the chip folds them in registers.
+Each case runs a batch large enough for the second and every request alone (the first), which must give the same bits,
+and checks the batch against the float64 oracle.  Sizes: one tile, ends inside the first unit, block and split and just
+past them, fewer tiles than waves, more requests than one scan of the lengths holds, and both row-block forms."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from judge import normalised_error as nerr
+from vmk.ops import decode, decode_paged, spec
+
+pytestmark = pytest.mark.gpu
+
+DECODE = [dict(B=70, L=40, L_min=1), dict(B=9, L=2049), dict(B=12, L=4096, L_min=1), dict(B=33, L=1025, L_min=1),
+          dict(B=40, L=513, Hq=8, Hkv=1), dict(B=9, L=2500, L_min=1, Hq=64, Hkv=8, dtype="bf16"),
+          dict(B=24, L=6000, L_min=1, Hq=48, Hkv=2)]
+PAGED = [dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16")]
+SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16), dict(B=9, L=300, k=11, Hq=8, Hkv=2),
+        dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9)]
+
+
+def same_bits(a, b):
+    return torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+def check(out, ref):
+    torch.cuda.synchronize()
+    em, _ = nerr(out.float().cpu().numpy().astype(np.float64), ref)
+    print(f"  err max {em:.3e}", flush=True)
+    # 16-bit results of values below 5: half a unit of the last place is 2^-9 of the value in bf16, 2^-12 in fp16; P and
+    # the partials round at the same precision, so the sum stays within four of them.
+    assert em <= (4 * 2.0 ** -9 if out.dtype == torch.bfloat16 else 4 * 2.0 ** -12)
+
+
+@pytest.mark.parametrize("shape", DECODE)
+def test_decode_batch_equals_requests_alone(shape):
+    import vmk
+    print(f"decode {shape}", flush=True)
+    inp = decode.make_inputs(shape, seed=41, device="cuda")
+    out = vmk.decode(**inp)
+    for i in range(shape["B"]):
+        assert same_bits(vmk.decode(**decode.row_inputs(inp, i))[0], out[i]), i
+    check(out, oracle.decode.ref64(**inp))
+
+
+@pytest.mark.parametrize("shape", PAGED)
+def test_paged_decode_batch_equals_requests_alone(shape):
+    import vmk
+    print(f"decode_paged {shape}", flush=True)
+    inp = decode_paged.make_inputs(shape, seed=42, device="cuda")
+    out = vmk.decode_paged(**inp)
+    for i in range(shape["B"]):
+        assert same_bits(vmk.decode_paged(**decode_paged.row_inputs(inp, i))[0], out[i]), i
+    check(out, oracle.decode_paged.ref64(**inp))
+
+
+@pytest.mark.parametrize("shape", SPEC)
+def test_verify_batch_equals_requests_alone(shape):
+    import spec_mi355x
+    print(f"spec {shape}", flush=True)
+    inp = spec.make_inputs(shape, seed=43, dist="chain", device="cuda")
+    out = spec_mi355x.kernel(**inp)
+    for i in range(shape["B"]):
+        assert same_bits(spec_mi355x.kernel(**spec.row_inputs(inp, i))[0], out[i]), i
+    check(out, oracle.spec.ref64(**inp))

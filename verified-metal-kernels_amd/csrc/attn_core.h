@@ -479,11 +479,14 @@ __device__ __forceinline__ void ring_walk(char* ring, const Src& src, int kbeg, 
 // The key source `src` provides: ktile(key0) / vtile(key0) (the first of the 32 K / V rows of the tile starting at
 // key0, a multiple of 32 from the range start; rows at or past kend are not read; the rows are 256 bytes apart, or
 // src.row_bytes(key0) apart when Src::kStrided), kend, scale (log2-domain softmax scale) and mask(s, key0, g)
-// (masked scores of the raw S^T tile -> -inf).
-template <int NS, class Src, class V>
+// (masked scores of the raw S^T tile -> -inf).  after(j) runs when j tiles have been computed and more follow.
+struct NoAfter {
+  __device__ __forceinline__ void operator()(int) const {}
+};
+template <int NS, class Src, class V, class After = NoAfter>
 __device__ __forceinline__ void wave_walk(RowState& st, const V (&qb)[8], char* __restrict__ ring,
                                           const char* __restrict__ base, const TileLanes& tl, const Src& src,
-                                          int kbeg, int t0, int ntiles, int tstep, int lane) {
+                                          int kbeg, int t0, int ntiles, int tstep, int lane, After after = After()) {
   static_assert(NS >= 2 && NS <= 4, "1 to 3 tiles in flight");
   if (t0 >= ntiles) return;
   const int n = (ntiles - t0 + tstep - 1) / tstep;          // tiles of this wave
@@ -503,11 +506,72 @@ __device__ __forceinline__ void wave_walk(RowState& st, const V (&qb)[8], char* 
       if (jn < n) issue_tile_dma(ring + ((S + NS - 1) % NS) * kStageBytes, src, key_of(jn), tl, lane);
       wait_vmem_dyn(16 * min(NS - 1, n - 1 - j));
       compute_tile_lds(st, qb, base + S * kStageBytes, tl, src, key_of(j), lane);
+      if (j + 1 < n) after(j + 1);
       return true;
     };
     if (!unroll_while<0, NS>(step)) break;
   }
 }
+
+// ---- folding the states of consecutive units of keys.  A unit's state becomes (O, m, l) with l the row's whole sum
+// (equal in both lane halves); the fold of two, and the merge of the interleaving waves' states that follows, are
+// written out with their roundings (merge_add), so that they give the same bits wherever they run: in a wave's
+// registers, or in a combine launch over stored units.
+__device__ __forceinline__ float merge_scale(float m, float M) { return fast_exp2(m - (M == kNegInf ? 0.f : M)); }
+// acc + a * x, rounded once.
+__device__ __forceinline__ float merge_add(float acc, float a, float x) { return __builtin_fmaf(a, x, acc); }
+// ah * h + au * u, the second product rounded first.
+__device__ __forceinline__ float fold_val(float ah, float h, float au, float u) {
+#pragma clang fp contract(off)
+  const float t = au * u;
+  return __builtin_fmaf(ah, h, t);
+}
+
+// The folded units so far, kept in AGPRs: they are touched once a unit, and a wave of these walks has its SIMD to
+// itself (128 KB of LDS), so the accumulation registers are free, while its VGPRs are nearly all in use.
+struct HeldState {
+  float o[64], m, l;
+  __device__ __forceinline__ static void put(float& slot, float v) {
+    asm("" : "+a"(v));                                      // the compiler's own copy into an AGPR
+    slot = v;
+  }
+  // Keeps the values in AGPRs across the tile loop (a value in a VGPR at the loop's end would be copied every turn).
+  __device__ __forceinline__ void pin() {
+#pragma unroll
+    for (int i = 0; i < 64; ++i) asm volatile("" : "+a"(o[i]));
+  }
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < 64; ++i) put(o[i], 0.f);
+    m = kNegInf;
+    l = 0.f;
+  }
+  // Takes a unit's state: the first one as it is, later ones folded in.
+  __device__ __forceinline__ void take(const RowState& st, bool first) {
+    const float ul = st.l + xor32(st.l);
+    if (first) {
+#pragma unroll
+      for (int i = 0; i < 64; ++i) put(o[i], st.o[i >> 4][i & 15]);
+      m = st.m;
+      l = ul;
+      return;
+    }
+    const float M = fmaxf(m, st.m), ah = merge_scale(m, M), au = merge_scale(st.m, M);
+#pragma unroll
+    for (int i = 0; i < 64; ++i) put(o[i], fold_val(ah, o[i], au, st.o[i >> 4][i & 15]));
+    l = fold_val(ah, l, au, ul);
+    m = M;
+  }
+  // The last unit folded in, into st (whose l becomes the row's whole sum).
+  __device__ __forceinline__ void finish(RowState& st) const {
+    const float ul = st.l + xor32(st.l);
+    const float M = fmaxf(m, st.m), ah = merge_scale(m, M), au = merge_scale(st.m, M);
+#pragma unroll
+    for (int i = 0; i < 64; ++i) st.o[i >> 4][i & 15] = fold_val(ah, o[i], au, st.o[i >> 4][i & 15]);
+    st.l = fold_val(ah, l, au, ul);
+    st.m = M;
+  }
+};
 
 // ---- paged caches
 // Keys [kbeg, kend) of one KV head of a sequence in a paged cache: pages of ps rows (ps a multiple of 32, so a tile
@@ -562,8 +626,9 @@ __device__ __forceinline__ PagedSrc<kNHD> paged_src(const f16* kpool, const f16*
   s.rb_page = (uint32_t)Hkv * 256u;
   const int key = kbeg + kTile * (int)(threadIdx.x & 63);     // this lane's tile
   const int slot = key / ps;
-  const int page = key < kend && slot < ntable ? table[slot] : -1;
-  s.here = (unsigned)page < (unsigned)num_pages;
+  // The table entry is loaded whether or not the key is in use, so that the load does not wait for a length.
+  const int page = slot < ntable ? table[slot] : -1;
+  s.here = key < kend && (unsigned)page < (unsigned)num_pages;
   const size_t row = key - slot * ps;                        // the tile's first row within its page
   const size_t off = (kNHD ? ((size_t)page * ps + row) * Hkv + h : ((size_t)page * Hkv + h) * ps + row) * 128;
   s.kt = s.here ? kpool + off : g_zero_tile;
@@ -624,10 +689,11 @@ constexpr int kAttnSmemBytes = 8 * kStageBytes;
 constexpr int kAttnSlotsEnd = 4 * kSlotBytes;
 static_assert(kAttnSlotsEnd <= kAttnSmemBytes, "merge slots must fit in the stage memory");
 
-template <int WR, int WK, int NSW = 2, class V = half8, class Src, class QRow, class PT>
+// kFold: a wave's tiles go in units of `unit` tiles (a power of two), each with a state of its own, folded in order.
+template <int WR, int WK, int NSW = 2, class V = half8, bool kFold = false, class Src, class QRow, class PT>
 __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow, int nrows, int kbeg, int ntiles,
-                                          PT* po, float* pml) {
-  static_assert(WR * WK == 4 && WR * WK * NSW <= 8, "four waves, rings within the stage memory");
+                                          PT* po, float* pml, int unit = 0) {
+  static_assert(WR * WK == 4 && WK > 1 && WR * WK * NSW <= 8, "four waves, rings within the stage memory");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave % WR, wk = wave / WR;
   const int r = lane & 31, g = lane >> 5;
@@ -638,13 +704,31 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
   row_state_init(st);
   const uint32_t ring_off = (uint32_t)wave * NSW * kStageBytes;
   const TileLanes tl = tile_lanes(lane, ring_off);
-  wave_walk<NSW>(st, qb, smem + ring_off, smem, tl, src, kbeg, wk, ntiles, WK, lane);
+  if constexpr (kFold) {
+    if (ntiles <= 0) return;                                // the whole workgroup: the merge does not look here
+    HeldState held;
+    bool first = true;
+    held.clear();
+    wave_walk<NSW>(st, qb, smem + ring_off, smem, tl, src, kbeg, wk, ntiles, WK, lane, [&](int j) {
+      held.pin();
+      if ((j & (unit - 1)) == 0) {
+        held.take(st, first);
+        first = false;
+        row_state_init(st);
+      }
+    });
+    if (first)
+      st.l += xor32(st.l);
+    else
+      held.finish(st);
+  } else {
+    wave_walk<NSW>(st, qb, smem + ring_off, smem, tl, src, kbeg, wk, ntiles, WK, lane);
+    st.l += xor32(st.l);
+  }
   const int nvalid = nrows - wr * 32;
   PT* pob = po + (size_t)wr * 32 * 128;
   float* pmlb = pml + wr * 32 * 2;
-  if constexpr (WK == 1) {
-    store_partial(pob, pmlb, st, lane, nvalid);
-  } else {
+  {
     __syncthreads();                                        // every walk is done: the rings become slots
     state_to_slot(smem + wave * kSlotBytes, st, lane);
     __syncthreads();
@@ -655,14 +739,13 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
       mk[k] = ml.x;
       M = fmaxf(M, ml.x);
     }
-    const float muse = (M == kNegInf) ? 0.f : M;
-    float ak[WK], l = 0.f;
+    float ak[WK], ltot = 0.f;
 #pragma unroll
     for (int k = 0; k < WK; ++k) {
-      ak[k] = fast_exp2(mk[k] - muse);
-      l += ak[k] * reinterpret_cast<const float2*>(smem + (k * WR + wr) * kSlotBytes + 64 * 64 * 4)[lane].y;
+      ak[k] = merge_scale(mk[k], M);
+      ltot = merge_add(ltot, ak[k],
+                       reinterpret_cast<const float2*>(smem + (k * WR + wr) * kSlotBytes + 64 * 64 * 4)[lane].y);
     }
-    const float ltot = l + xor32(l);
     const float inv = part_inv(ltot);
 #pragma unroll
     for (int j = 0; j < 4 / WK; ++j) {
@@ -674,7 +757,11 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
       for (int k = 0; k < WK; ++k) {
         const floatx4* o = reinterpret_cast<const floatx4*>(smem + (k * WR + wr) * kSlotBytes);
 #pragma unroll
-        for (int blk = 0; blk < 4; ++blk) acc[blk] += ak[k] * o[(dt * 4 + blk) * 64 + lane];
+        for (int blk = 0; blk < 4; ++blk) {
+          const floatx4 x = o[(dt * 4 + blk) * 64 + lane];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[blk][c] = merge_add(acc[blk][c], ak[k], x[c]);
+        }
       }
       if (r < nvalid)
 #pragma unroll

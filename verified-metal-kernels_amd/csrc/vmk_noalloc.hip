@@ -64,5 +64,6 @@ extern "C" int vmk_spec_verify_noalloc(const void* q, const void* k, const void*
   }
   void* partials = nullptr;
   if (int rc = scratch_address((hipStream_t)stream, &partials)) return rc;
-  return spec_noalloc_launch(q, k, v, mask_words, out, B, kd, Hq, Hkv, L, W, partials, (hipStream_t)stream);
+  return spec_noalloc_launch(q, k, v, mask_words, out, B, kd, Hq, Hkv, L, W, partials, kScratchBytes,
+                             (hipStream_t)stream);
 }

@@ -3,12 +3,11 @@
 // Replaces the reference's spec_verify_qperm / spec_verify_partial_mpp / spec_verify_combine Metal kernels
 // (kernels/spec_opus55_v7.py:186-199, 228-342, 344-365) behind the kernel(q, k, v, bits) contract of
 // ops/spec.py:1-3.  The draft mask is applied in registers from (B, kd, W) 32-bit words, so kd is not limited to 32.
-#include "attn_core.h"
-#include "vmk_internal.h"
-
+#include "key_split.h"
 
 namespace vmk {
 
+// The row split's arguments (more than 64 query rows per KV head); the key split's are KeySplitArgs.
 struct SpecArgs {
   const f16* q;            // (B, kd, Hq, 128)
   const f16* k;            // (B, Hkv, L, 128)
@@ -19,50 +18,21 @@ struct SpecArgs {
   float* part_ml;          // [item][32*WR][2]
   f16* out;                // (B, kd, Hq, 128)
   int B, kd, Hq, Hkv, G, L, W;
-  int WR, WK, nrb, nsplit, chunk;
+  int WR, nrb, nsplit, chunk;
   float sl2;               // softmax scale * log2(e)
-  // Paged decode: k, v are the page pools (num_pages pages of ps rows, HND or NHD), pages the (B, max_pages) table.
-  const int* pages;
-  int ps, max_pages, num_pages;
 };
 
 // Keys of one (batch, KV head) for one split: rows of k/v, and the draft mask of this lane's row on the last kd
-// positions, preloaded as up to kMaskWords 32-bit words (kd <= 32 * kMaskWords).
-constexpr int kMaskWords = 8;
-
-typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-
-// The mask words are a vector value, not an array: an array member makes the compiler keep the whole struct in LDS
-// and fetch the words one dependent round trip at a time before the first tile.
+// positions.
 struct SpecSrc {
   const f16* kbase;
   const f16* vbase;
-  u32x8 mw;          // the row's mask words; words at or past nw are not used
-  int nw, kend, tail0;
+  DraftMask dm;
+  int kend, tail0;
   float scale;
   static constexpr bool kStrided = false;   // rows 256 bytes apart
   __device__ const f16* ktile(int key0) const { return kbase + (size_t)key0 * 128; }
   __device__ const f16* vtile(int key0) const { return vbase + (size_t)key0 * 128; }
-  __device__ uint32_t bit(int j) const {          // bit j of the row's mask, 0 <= j < 32 * kMaskWords
-    const int wi = j >> 5;
-    uint32_t w = mw[0];
-#pragma unroll
-    for (int i = 1; i < kMaskWords; ++i) w = wi == i ? mw[i] : w;
-    return wi < nw ? (w >> (j & 31)) & 1u : 0u;
-  }
-  // Loads the nw (1 .. kMaskWords) mask words at mrow; every address stays inside the row.  mrow == null: the whole
-  // tail is visible.
-  __device__ void load_mask(const uint32_t* mrow, int n) {
-    if (!mrow) {
-      nw = kMaskWords;
-#pragma unroll
-      for (int i = 0; i < kMaskWords; ++i) mw[i] = ~0u;
-      return;
-    }
-    nw = n;
-#pragma unroll
-    for (int i = 0; i < kMaskWords; ++i) mw[i] = ldg4(mrow + min(i, n - 1));
-  }
   __device__ void mask(floatx16& s, int key0, int g) const {
     if (key0 + kTile <= tail0 && key0 + kTile <= kend) return;   // whole tile visible (same for the whole wave)
 #pragma unroll
@@ -70,7 +40,7 @@ struct SpecSrc {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const int key = key0 + 8 * blk + 4 * g + c;
-        const uint32_t vis = (key < tail0) | bit(max(key - tail0, 0));
+        const uint32_t vis = (key < tail0) | dm.bit(max(key - tail0, 0));
         const bool ok = (key < kend) & (vis != 0u);
         s[4 * blk + c] = ok ? s[4 * blk + c] : kNegInf;
       }
@@ -80,68 +50,6 @@ struct SpecSrc {
 // Cache positions of batch entry b: lens[b] clamped to [kd, L] (the query rows are the last kd of them), or L.
 __device__ __forceinline__ int batch_len(const SpecArgs& a, int b) {
   return a.lens ? min(max(a.lens[b], a.kd), a.L) : a.L;
-}
-
-// One workgroup = WR x WK waves: WR row blocks of 32 rows, WK waves interleaving the key tiles of one split.
-// V is the operand type: half8 (fp16 inputs) or bf16x8 (bf16 inputs).
-template <class V>
-__global__ __launch_bounds__(256) void spec_partial_kernel(SpecArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[kAttnSmemBytes];
-  const int item = blockIdx.x;
-  const int split = item % a.nsplit;
-  const int rb = (item / a.nsplit) % a.nrb;
-  const int grp = item / (a.nsplit * a.nrb);
-  const int b = grp / a.Hkv, h = grp % a.Hkv;
-  const int R = a.kd * a.G;
-  const int row0 = rb * a.WR * 32;                        // first query row (i*G + gg) of this workgroup
-  const int lrow = row0 + (threadIdx.x & 31) + 32 * ((threadIdx.x >> 6) % a.WR);
-  const int di = (lrow < R ? lrow : 0) / a.G;
-
-  SpecSrc src;
-  const size_t kvoff = (size_t)grp * a.L * 128;
-  src.kbase = a.k + kvoff;
-  src.vbase = a.v + kvoff;
-  src.load_mask(a.bits ? a.bits + (size_t)(b * a.kd + di) * a.W : nullptr, a.W);
-  const int Lb = batch_len(a, b);
-  const int kbeg = split * a.chunk;
-  src.kend = min(Lb, kbeg + a.chunk);
-  src.tail0 = Lb - a.kd;
-  src.scale = a.sl2;
-  const int ntiles = max(0, (src.kend - kbeg + kTile - 1) / kTile);
-  const size_t rows_wg = 32 * a.WR;
-  auto qrow = [&](int r) {
-    const int qr = row0 + r, i = qr / a.G, gg = qr % a.G;
-    return a.q + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
-  };
-  part_t<elem_t<V>>* po = reinterpret_cast<part_t<elem_t<V>>*>(a.part_o) + (size_t)item * rows_wg * 128;
-  float* pml = a.part_ml + (size_t)item * rows_wg * 2;
-  if (a.WK == 4)
-    attend_wg<1, 4, 2, V>(smem, src, qrow, R - row0, kbeg, ntiles, po, pml);
-  else
-    attend_wg<2, 2, 2, V>(smem, src, qrow, R - row0, kbeg, ntiles, po, pml);
-}
-
-// Paged single-token decode: the key-split kernel with request b's keys [0, lens[b]) read through its page table
-// (paged_src; a split holds at most 2048 keys, the decode split size up to 16 query heads per KV head).  Absent
-// pages are left out of the softmax.  With every page present the partials are those of spec_partial_kernel on the
-// gathered cache, so the output is bit-equal to vmk_decode's.
-template <bool kNHD, class V>
-__global__ __launch_bounds__(256) void decode_paged_kernel(SpecArgs a) {
-  __shared__ __attribute__((aligned(16))) char smem[kAttnSmemBytes];
-  const int item = blockIdx.x;
-  const int split = item % a.nsplit;
-  const int grp = item / a.nsplit;                         // one row block: G <= 16 rows
-  const int b = grp / a.Hkv, h = grp % a.Hkv;
-  const int Lb = batch_len(a, b);
-  const int kbeg = split * a.chunk;
-  const int kend = min(Lb, kbeg + a.chunk);
-  const int ntiles = max(0, (kend - kbeg + kTile - 1) / kTile);
-  const PagedSrc<kNHD> src = paged_src<kNHD>(a.k, a.v, a.ps, a.Hkv, a.num_pages, a.sl2,
-                                             a.pages + (size_t)b * a.max_pages, a.max_pages, h, kbeg, kend);
-  auto qrow = [&](int r) { return a.q + ((size_t)b * a.Hq + h * a.G + r) * 128; };
-  part_t<elem_t<V>>* po = reinterpret_cast<part_t<elem_t<V>>*>(a.part_o) + (size_t)item * 32 * 128;
-  float* pml = a.part_ml + (size_t)item * 32 * 2;
-  attend_wg<1, 4, 2, V>(smem, src, qrow, a.G, kbeg, ntiles, po, pml);
 }
 
 // Row-split variant for kd*G > 64 rows: NW waves own 32 rows each and share one LDS ring, so every K/V tile of the
@@ -162,7 +70,7 @@ __global__ __launch_bounds__(64 * NW) void spec_partial_rows_kernel(SpecArgs a) 
   const size_t kvoff = (size_t)grp * a.L * 128;
   src.kbase = a.k + kvoff;
   src.vbase = a.v + kvoff;
-  src.load_mask(a.bits ? a.bits + (size_t)(b * a.kd + di) * a.W : nullptr, a.W);
+  src.dm.load(a.bits ? a.bits + (size_t)(b * a.kd + di) * a.W : nullptr, a.W);
   const int Lb = batch_len(a, b);
   const int kbeg = split * a.chunk;
   src.kend = min(Lb, kbeg + a.chunk);
@@ -238,28 +146,26 @@ static void launch_spec_combine(const SpecArgs& a, int64_t rows, hipStream_t s) 
     hipLaunchKernelGGL(spec_combine_kernel<E>, dim3((unsigned)rows), dim3(128), 0, s, a);
 }
 
+// The row split's plan.
 struct SpecPlan {
-  bool rows_mode;
-  int WR, WK, nrb, nsplit, chunk;
+  int WR, nrb, nsplit, chunk;
   size_t po_floats, pml_floats;
 };
+
+// More than 64 query rows per KV head take the row split, whose waves share each tile; the others the key split.
+static bool spec_rows_mode(int64_t rows) { return rows > 64; }
 
 static SpecPlan spec_plan(int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_t L) {
   SpecPlan p;
   const int64_t G = Hq / Hkv, R = kd * G;
-  p.rows_mode = R > 64;
-  if (p.rows_mode) { p.WR = R <= 128 ? 4 : 8; p.WK = 1; }   // row-split: WR = waves sharing one ring
-  else if (R <= 32) { p.WR = 1; p.WK = 4; }
-  else { p.WR = 2; p.WK = 2; }
+  p.WR = R <= 128 ? 4 : 8;                                  // waves sharing one ring
   const int64_t rows_wg = 32 * p.WR;
   p.nrb = (int)((R + rows_wg - 1) / rows_wg);
   const int64_t base = B * Hkv * p.nrb;
   // The split size depends on the rows of one group (kd * G) only, never on B: a batch entry goes through the same
-  // key splits, tile order and merge as the same entry alone, so its rows are bit-equal (batch invariance).  Key
-  // split: 2048 keys up to 16 rows (decode: 256 workgroups once B * Hkv * L reaches 2^19), then 128 keys per row
-  // (C3: 4096), which keeps the fp32 partials at 1/64 of the K/V bytes.  Row split: 4096 keys, 16 per row beyond.
-  const int64_t chunk = p.rows_mode ? std::max<int64_t>(4096, 16 * R)
-                                    : std::min<int64_t>(8192, std::max<int64_t>(2048, 128 * R));
+  // key splits, tile order and merge as the same entry alone, so its rows are bit-equal (batch invariance).  4096
+  // keys, 16 per row beyond.
+  const int64_t chunk = std::max<int64_t>(4096, 16 * R);
   p.chunk = (int)chunk;
   p.nsplit = (int)((L + chunk - 1) / chunk);
   const size_t items = (size_t)base * p.nsplit;
@@ -268,39 +174,37 @@ static SpecPlan spec_plan(int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_
   return p;
 }
 
+// Partials of the row split: the normalised O rows in the partial type of V's inputs, then the (m, l) pairs from the
+// next 256-byte boundary.  Every partial the combine reads is written first, so the region needs no initialisation.
+template <class V>
+static size_t spec_ml_offset(const SpecPlan& p) {
+  return (p.po_floats * sizeof(part_t<elem_t<V>>) + 255) / 256 * 256;
+}
+
 }  // namespace vmk
 
 using namespace vmk;
 
 extern "C" size_t vmk_spec_workspace_size(int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_t D, int64_t L) {
   if (B <= 0 || kd <= 0 || Hkv <= 0 || Hq % Hkv || D != 128 || L < kd) return 0;
+  const int64_t R = kd * (Hq / Hkv);
+  if (!spec_rows_mode(R))
+    return kWsHead + key_split_bytes(key_split_plan(B * Hkv, R, L), B * Hkv, sizeof(float)) + 512;
   SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
   return kWsHead + (p.po_floats + p.pml_floats) * sizeof(float) + 512;   // fits either partial type
 }
 
-// Partial launch (key split or row split by the plan) and LSE-combine launch of one spec/decode call; V is the
-// operand type of the inputs (half8: fp16, bf16x8: bf16).  `partials` is the 256-byte aligned region of
-// spec_partials_bytes<V>(p) bytes that receives the partials: every partial the combine reads is written first, so
-// the region needs no initialisation.  Layout: the normalised O rows in the partial type of V's inputs, then the
-// (m, l) pairs from the next 256-byte boundary.
+// Partial launch (row split) and LSE-combine launch of one spec/decode call; V is the operand type of the inputs
+// (half8: fp16, bf16x8: bf16).  `partials`: 256-byte aligned.
 template <class V>
-static size_t spec_ml_offset(const SpecPlan& p) {
-  return (p.po_floats * sizeof(part_t<elem_t<V>>) + 255) / 256 * 256;
-}
-template <class V>
-static size_t spec_partials_bytes(const SpecPlan& p) { return spec_ml_offset<V>(p) + p.pml_floats * sizeof(float); }
-
-template <class V>
-static int spec_launch(SpecArgs& a, const SpecPlan& p, void* partials, hipStream_t s) {
+static int spec_rows_launch(SpecArgs& a, const SpecPlan& p, void* partials, hipStream_t s) {
   a.part_o = partials;
   a.part_ml = reinterpret_cast<float*>((char*)partials + spec_ml_offset<V>(p));
-  a.WR = p.WR; a.WK = p.WK; a.nrb = p.nrb; a.nsplit = p.nsplit; a.chunk = p.chunk;
+  a.WR = p.WR; a.nrb = p.nrb; a.nsplit = p.nsplit; a.chunk = p.chunk;
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
   const unsigned items = (unsigned)(a.B * a.Hkv * p.nrb * p.nsplit);
   prof_before(kKSpecPartial, s);
-  if (!p.rows_mode)
-    hipLaunchKernelGGL(spec_partial_kernel<V>, dim3(items), dim3(256), 0, s, a);
-  else if (p.WR == 4)
+  if (p.WR == 4)
     hipLaunchKernelGGL((spec_partial_rows_kernel<4, V>), dim3(items), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL((spec_partial_rows_kernel<8, V>), dim3(items), dim3(512), 0, s, a);
@@ -310,6 +214,44 @@ static int spec_launch(SpecArgs& a, const SpecPlan& p, void* partials, hipStream
   launch_spec_combine<elem_t<V>>(a, (int64_t)a.B * a.Hkv * a.kd * a.G, s);
   prof_after(kKSpecCombine, s);
   VMK_CHECK_HIP(hipGetLastError());
+  return 0;
+}
+
+// One spec or decode call over contiguous caches, key split or row split by its rows per KV head.  Partials go to
+// `partials` (256-byte aligned); budget: with more groups than its bytes hold partials for, the key split goes through
+// the groups in several launches (0: no limit).
+template <class V>
+static int spec_call(const void* q, const void* k, const void* v, const void* mask_words, const void* lens, void* out,
+                     int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_t L, int64_t W, void* partials,
+                     size_t budget, hipStream_t s) {
+  const int64_t G = Hq / Hkv, R = kd * G;
+  if (spec_rows_mode(R)) {
+    SpecArgs a;
+    a.q = (const f16*)q; a.k = (const f16*)k; a.v = (const f16*)v; a.bits = (const uint32_t*)mask_words;
+    a.lens = (const int*)lens;
+    a.out = (f16*)out;
+    a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)G; a.L = (int)L; a.W = (int)W;
+    return spec_rows_launch<V>(a, spec_plan(B, kd, Hq, Hkv, L), partials, s);
+  }
+  KeySplitArgs a = {};
+  a.q = (const f16*)q; a.k = (const f16*)k; a.v = (const f16*)v; a.bits = (const uint32_t*)mask_words;
+  a.lens = (const int*)lens;
+  a.out = out;
+  a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)G; a.L = (int)L; a.W = (int)W;
+  a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
+  const int64_t groups = B * Hkv;
+  const KeySplitPlan p = key_split_plan(groups, R, L);
+  int64_t step = groups;
+  if (budget)
+    step = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(budget / (key_split_bytes(p, 1, sizeof(part_t<elem_t<V>>)) + 256))));
+  for (int64_t g0 = 0; g0 < groups; g0 += step) {
+    a.g0 = (int)g0;
+    a.ngrp = (int)std::min(step, groups - g0);
+    // The masked kernels serve decode with more than 32 rows, too (no mask words: every position visible).
+    const int rc = a.bits || R > 32 ? key_split_launch<kStreamContig, true, V>(a, p, partials, s)
+                                    : key_split_launch<kStreamContig, false, V>(a, p, partials, s);
+    if (rc) return rc;
+  }
   return 0;
 }
 
@@ -334,13 +276,8 @@ static int spec_verify(const void* q, const void* k, const void* v, const void* 
   if (int rc = spec_check_args(q, k, v, mask_words, out, B, kd, Hq, Hkv, D, L, W)) return rc;
   const size_t need = vmk_spec_workspace_size(B, kd, Hq, Hkv, D, L);
   VMK_CHECK(workspace && ws_bytes >= need, "workspace too small (query vmk_spec_workspace_size)");
-  SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
-  SpecArgs a;
-  a.q = (const f16*)q; a.k = (const f16*)k; a.v = (const f16*)v; a.bits = (const uint32_t*)mask_words;
-  a.lens = nullptr;
-  a.out = (f16*)out;
-  a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.L = (int)L; a.W = (int)W;
-  return spec_launch<V>(a, p, align_up((char*)workspace + kWsHead, 256), (hipStream_t)stream);
+  return spec_call<V>(q, k, v, mask_words, nullptr, out, B, kd, Hq, Hkv, L, W,
+                      align_up((char*)workspace + kWsHead, 256), 0, (hipStream_t)stream);
 }
 
 // Plain single-token decode: the verify path with one query row per request and no mask (the row's own position is
@@ -360,13 +297,8 @@ static int decode(const void* q, const void* k, const void* v, const void* lens,
   VMK_CHECK(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out), "tensors must be 16-byte aligned");
   const size_t need = vmk_decode_workspace_size(B, Hq, Hkv, D, L);
   VMK_CHECK(workspace && ws_bytes >= need, "workspace too small (query vmk_decode_workspace_size)");
-  SpecPlan p = spec_plan(B, 1, Hq, Hkv, L);
-  SpecArgs a;
-  a.q = (const f16*)q; a.k = (const f16*)k; a.v = (const f16*)v; a.bits = nullptr;
-  a.lens = (const int*)lens;
-  a.out = (f16*)out;
-  a.B = (int)B; a.kd = 1; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.L = (int)L; a.W = 1;
-  return spec_launch<V>(a, p, align_up((char*)workspace + kWsHead, 256), (hipStream_t)stream);
+  return spec_call<V>(q, k, v, nullptr, lens, out, B, 1, Hq, Hkv, L, 1, align_up((char*)workspace + kWsHead, 256), 0,
+                      (hipStream_t)stream);
 }
 
 extern "C" int vmk_spec_verify(const void* q, const void* k, const void* v, const void* mask_words, void* out,
@@ -420,29 +352,18 @@ static int decode_paged(const void* q, const void* k_pages, const void* v_pages,
   const int64_t L = page_size * max_pages;
   const size_t need = vmk_decode_paged_workspace_size(B, Hq, Hkv, D, page_size, max_pages);
   VMK_CHECK(workspace && ws_bytes >= need, "workspace too small (query vmk_decode_paged_workspace_size)");
-  SpecPlan p = spec_plan(B, 1, Hq, Hkv, L);
-  VMK_CHECK(!p.rows_mode && p.WR == 1 && p.WK == 4 && p.nrb == 1 && p.chunk <= 2048, "unsupported decode plan");
-  SpecArgs a;
-  a.q = (const f16*)q; a.k = (const f16*)k_pages; a.v = (const f16*)v_pages; a.bits = nullptr;
+  KeySplitArgs a = {};
+  a.q = (const f16*)q; a.k = (const f16*)k_pages; a.v = (const f16*)v_pages;
   a.lens = (const int*)lens;
-  a.out = (f16*)out;
-  a.B = (int)B; a.kd = 1; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.L = (int)L; a.W = 1;
   a.pages = (const int*)page_table;
+  a.out = out;
+  a.B = (int)B; a.kd = 1; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.L = (int)L; a.W = 1;
   a.ps = (int)page_size; a.max_pages = (int)max_pages; a.num_pages = (int)num_pages;
-  a.part_o = align_up((char*)workspace + kWsHead, 256);
-  a.part_ml = reinterpret_cast<float*>((char*)a.part_o + spec_ml_offset<V>(p));
-  a.WR = p.WR; a.WK = p.WK; a.nrb = p.nrb; a.nsplit = p.nsplit; a.chunk = p.chunk;
+  a.ngrp = (int)(B * Hkv);
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
-  hipStream_t s = (hipStream_t)stream;
-  prof_before(kKSpecPartial, s);
-  hipLaunchKernelGGL((decode_paged_kernel<kNHD, V>), dim3((unsigned)(B * Hkv * p.nsplit)), dim3(256), 0, s, a);
-  prof_after(kKSpecPartial, s);
-  VMK_CHECK_HIP(hipGetLastError());
-  prof_before(kKSpecCombine, s);
-  launch_spec_combine<elem_t<V>>(a, B * Hq, s);
-  prof_after(kKSpecCombine, s);
-  VMK_CHECK_HIP(hipGetLastError());
-  return 0;
+  return key_split_launch<kNHD ? kStreamNHD : kStreamHND, false, V>(a, key_split_plan(B * Hkv, a.G, L),
+                                                                    align_up((char*)workspace + kWsHead, 256),
+                                                                    (hipStream_t)stream);
 }
 
 #define VMK_DECODE_PAGED_ENTRY(name, nhd, V)                                                                      \
@@ -464,21 +385,27 @@ VMK_DECODE_PAGED_ENTRY(vmk_decode_paged_nhd_bf16, true, bf16x8)
 // object of their own, which the HIP runtime loads onto a device (and so allocates the scratch on) only when the
 // scratch is first looked up there.
 namespace vmk {
+// The bytes a shape is accepted or refused by.  The key split's partials are not this many (its launches go through
+// the groups as the scratch holds them); its measure is one fp16 partial per 32 rows and split of 128 keys per row
+// (between 2048 and 8192), which callers have sized their shapes by.
 int spec_noalloc_need(const void* q, const void* k, const void* v, const void* mask_words, void* out, int64_t B,
                       int64_t kd, int64_t Hq, int64_t Hkv, int64_t D, int64_t L, int64_t W, size_t* need) {
   if (int rc = spec_check_args(q, k, v, mask_words, out, B, kd, Hq, Hkv, D, L, W)) return rc;
-  *need = spec_partials_bytes<half8>(spec_plan(B, kd, Hq, Hkv, L));
+  const int64_t R = kd * (Hq / Hkv);
+  if (spec_rows_mode(R)) {
+    const SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
+    *need = spec_ml_offset<half8>(p) + p.pml_floats * sizeof(float);
+  } else {
+    const int64_t chunk = std::min<int64_t>(8192, std::max<int64_t>(2048, 128 * R));
+    const size_t rows = (size_t)(B * Hkv) * ((L + chunk - 1) / chunk) * (R <= 32 ? 32 : 64);
+    *need = rows * (128 * sizeof(f16) + 2 * sizeof(float));
+  }
   return 0;
 }
 
 int spec_noalloc_launch(const void* q, const void* k, const void* v, const void* mask_words, void* out, int64_t B,
-                        int64_t kd, int64_t Hq, int64_t Hkv, int64_t L, int64_t W, void* partials, hipStream_t s) {
-  const SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
-  SpecArgs a;
-  a.q = (const f16*)q; a.k = (const f16*)k; a.v = (const f16*)v; a.bits = (const uint32_t*)mask_words;
-  a.lens = nullptr;
-  a.out = (f16*)out;
-  a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)(Hq / Hkv); a.L = (int)L; a.W = (int)W;
-  return spec_launch<half8>(a, p, partials, s);
+                        int64_t kd, int64_t Hq, int64_t Hkv, int64_t L, int64_t W, void* partials, size_t bytes,
+                        hipStream_t s) {
+  return spec_call<half8>(q, k, v, mask_words, nullptr, out, B, kd, Hq, Hkv, L, W, partials, bytes, s);
 }
 }  // namespace vmk
