@@ -1,4 +1,6 @@
-"""The two launches of the key split (decode and verification up to 64 rows per KV head): a call with few splits deals
+"""Calls that spread their work by the load of the chip give the same bits however it is spread.
+
+The key split (decode and verification up to 64 rows per KV head): a call with few splits deals
 units of keys out to all waves and folds them in its combine launch, a call that fills the chip folds them in registers.
 Each case runs a batch large enough for the second and every request alone (the first), which must give the same bits,
 and checks the batch against the float64 oracle.  Sizes: one tile, ends inside the first unit, block and split and just
@@ -9,7 +11,7 @@ import torch
 
 import oracle
 from judge import normalised_error as nerr
-from vmk.ops import decode, decode_paged, spec
+from vmk.ops import decode, decode_paged, prefix, prefix_paged, spec
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +21,13 @@ DECODE = [dict(B=70, L=40, L_min=1), dict(B=9, L=2049), dict(B=12, L=4096, L_min
 PAGED = [dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16")]
 SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16), dict(B=9, L=300, k=11, Hq=8, Hkv=2),
         dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9)]
+# Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone, which
+# is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows and of fewer
+# tiles than waves, and eight rows per KV head.
+PREFIX = [dict(N=24, P=8000, S=1000, S_min=0), dict(N=9, P=8191, S=1025, S_min=1), dict(N=13, P=7409, S=34),
+          dict(N=12, P=4100, S=500, S_min=0, Hq=64, dtype="bf16"), dict(N=20, P=5000, S=2048, S_min=1, Hq=16, Hkv=4)]
+PREFIX_PAGED = [dict(N=24, P=8192, S=1000, S_min=0, ps=64, dtype="bf16"),
+                dict(N=11, P=4704, S=700, S_min=0, ps=32, layout="NHD", Hq=64, absent=2)]
 
 
 def same_bits(a, b):
@@ -65,3 +74,25 @@ def test_verify_batch_equals_requests_alone(shape):
     for i in range(shape["B"]):
         assert same_bits(spec_mi355x.kernel(**spec.row_inputs(inp, i))[0], out[i]), i
     check(out, oracle.spec.ref64(**inp))
+
+
+@pytest.mark.parametrize("shape", PREFIX)
+def test_prefix_batch_equals_requests_alone(shape):
+    import vmk
+    print(f"prefix {shape}", flush=True)
+    inp = prefix.make_inputs(shape, seed=44, device="cuda")
+    out = vmk.prefix_decode(**inp)
+    for i in range(shape["N"]):
+        assert same_bits(vmk.prefix_decode(**prefix.row_inputs(inp, i))[0], out[i]), i
+    check(out, oracle.prefix.ref64(**inp))
+
+
+@pytest.mark.parametrize("shape", PREFIX_PAGED)
+def test_paged_prefix_batch_equals_requests_alone(shape):
+    import vmk
+    print(f"prefix_paged {shape}", flush=True)
+    inp = prefix_paged.make_inputs(shape, seed=45, device="cuda")
+    out = vmk.prefix_decode_paged(**inp)
+    for i in range(shape["N"]):
+        assert same_bits(vmk.prefix_decode_paged(**prefix_paged.row_inputs(inp, i))[0], out[i]), i
+    check(out, oracle.prefix_paged.ref64(**inp))

@@ -679,6 +679,21 @@ __device__ __forceinline__ void store_partial(PT* po, float* pml, const RowState
   }
 }
 
+// Writes one wave's state for its rows (< nvalid) of the 32 as it is, for a merge in fp32: the sums O (row stride 128)
+// and (m, l).
+__device__ __forceinline__ void store_sums(float* po, float* pml, const RowState& st, int lane, int nvalid) {
+  const int r = lane & 31, g = lane >> 5;
+  const float ltot = st.l + xor32(st.l);
+  if (r >= nvalid) return;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk)
+      store_part4(po + r * 128 + dt * 32 + 8 * blk + 4 * g,
+                  floatx4{st.o[dt][4 * blk], st.o[dt][4 * blk + 1], st.o[dt][4 * blk + 2], st.o[dt][4 * blk + 3]});
+  if (g == 0) *reinterpret_cast<float2*>(pml + 2 * r) = float2{st.m, ltot};
+}
+
 // ---- one workgroup of WR x WK waves (WR * WK = 4, 256 threads): WR row blocks of 32 rows, WK waves interleaving the
 // tiles of [kbeg, kbeg + 32*ntiles) through private rings of NSW stages.  Writes one partial (O, m, l) for the WG's
 // 32*WR rows to po (row stride 128 floats) / pml; rows >= nrows are skipped.  po/pml may point into smem past

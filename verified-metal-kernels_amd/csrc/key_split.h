@@ -280,20 +280,6 @@ __device__ __forceinline__ void land(V (&qb)[8]) {
   for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(qb[i]));
 }
 
-// Writes a unit's partial, the fp32 sums as they are, for its rows (< nvalid) of the 32.
-__device__ __forceinline__ void store_unit(float* po, float* pml, const RowState& st, int lane, int nvalid) {
-  const int r = lane & 31, g = lane >> 5;
-  const float ltot = st.l + xor32(st.l);
-  if (r >= nvalid) return;
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-    for (int blk = 0; blk < 4; ++blk)
-      store_part4(po + r * 128 + dt * 32 + 8 * blk + 4 * g,
-                  floatx4{st.o[dt][4 * blk], st.o[dt][4 * blk + 1], st.o[dt][4 * blk + 2], st.o[dt][4 * blk + 3]});
-  if (g == 0) *reinterpret_cast<float2*>(pml + 2 * r) = float2{st.m, ltot};
-}
-
 // One wave's part of a share: unit u of q in each of the blocks [beg, end), through its private ring of NS stages
 // (NS - 1 tiles in flight while one is computed).  At a unit's end the partial is stored and the state starts anew;
 // the ring runs on, its next tiles (of whatever unit or group) already requested.  The 16 O stores of a partial are
@@ -366,7 +352,7 @@ __device__ __forceinline__ void stream_walk(const KeySplitArgs& a, char* __restr
       --ahead;
       if (ct >= uend) {
         const size_t slot = ((size_t)(cg - a.g0) * a.nrb + rb) * a.slots + unit;
-        store_unit(reinterpret_cast<float*>(a.part_o) + slot * a.rows_s * 128, a.part_ml + slot * a.rows_s * 2, st, lane,
+        store_sums(reinterpret_cast<float*>(a.part_o) + slot * a.rows_s * 128, a.part_ml + slot * a.rows_s * 2, st, lane,
                    nvalid);
         stored = true;
         row_state_init(st);

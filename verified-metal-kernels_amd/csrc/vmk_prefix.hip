@@ -13,7 +13,8 @@
 // Launch 3 (prefix_combine_kernel, only when a suffix spans several chunks or there is no prefix): per output row,
 //   the log-sum-exp merge of its prefix and suffix partials.
 // With at most 128 rows per KV head, launches 1 and 2 are one grid (prefix_mixed_kernel; with at most 32 rows and
-// more items than CUs, its prefix items are single-wave units packed 2 or 4 per workgroup).  Its whole-suffix items
+// more items than CUs, its prefix items are single-wave units packed 2 or 4 per workgroup); when that grid has more
+// workgroups than CUs, single-wave workgroups and a merge launch (prefix_waves_kernel).  Its whole-suffix items
 // wait for their KV head's prefix partials and merge them in the same launch when G <= 4 and there are at most 32
 // prefix chunks (mfuse below); otherwise prefix_merge_kernel does the whole-suffix merges.
 #include "attn_core.h"
@@ -44,6 +45,7 @@ struct PrefixArgs {
   int fuse;                // 1: suffix items are whole suffixes and merge the (finished) prefix partials themselves
   int merge;               // 1: whole-suffix partials are merged with the prefix partials by prefix_merge_kernel
   int units;               // mixed launch, N*G <= 32: prefix units (one wave each) per workgroup; 0: row blocks
+  int n_wave_units;        // prefix_waves_kernel: its workgroups that are (or pad) prefix units
   int mfuse;               // 1: mixed launch whose whole-suffix items wait for their KV head's prefix partials and
                            //    merge them themselves (no merge launch)
   uint32_t* sync;          // mfuse: the sticky timeout flag, then per KV head the prefix arrivals and the finished
@@ -508,6 +510,135 @@ __global__ __launch_bounds__(256) void prefix_mixed_kernel(PrefixArgs a) {
   }
 }
 
+// Up to 128 rows per KV head and more items than the mixed launch runs in one round: the same work one wave at a time.
+// A workgroup is one wave with a two-stage ring (32 KB of LDS, so up to five share a CU and the dispatcher hands out the
+// next as each ends), and does a prefix unit (KV head, 32 of its N * G rows, prefix chunk) or a suffix piece (request,
+// KV head, one of the four interleaved tile sequences that a suffix item's waves walk).  With 128 KB workgroups a CU
+// holds one at a time, and a latency-bound prefix item and a suffix item ran one after the other.  Pieces are stored as
+// the walk leaves them (fp32 sums); prefix_waves_merge_kernel merges the four of a suffix as attend_wg does, and then
+// the prefix partials as every other path does, so the bits are theirs.  A chunk's row blocks run on one XCD (workgroup
+// id modulo 8), whose L2 then serves all but the first read of a tile.  Bound by latency (a tile takes a wave about
+// 1.1 us, a wave's start 4 us): N = 24, P = 8192 in pages, S <= 1000: 25.7 us and 5.4 for the merge, against 34.5 for the
+// mixed launch.  Three or four stages (three or two waves per CU) 32.9 and 43.5 us a call, five waves per CU (256
+// registers, spilled) 37.0, against 30.5.
+constexpr int kWaveStages = 2;
+template <int kPaged, class V>
+__global__ __launch_bounds__(64) void prefix_waves_kernel(PrefixArgs a) {
+  __shared__ __attribute__((aligned(16))) char smem[kWaveStages * kStageBytes];
+  const int lane = threadIdx.x, r = lane & 31;
+  const bool unit = (int)blockIdx.x < a.n_wave_units;
+  // What the wave walks: tiles t0, t0 + step, ... of keys [kbeg, kend) of one sequence, for nrows rows from row0 on.
+  int n, h, kbeg, kend, t0, step, row0, nrows, c = 0, piece = 0;
+  if (unit) {
+    // Chunk c = (slot / row blocks) * 8 + XCD, row block = slot % row blocks; ids past the last chunk do nothing.
+    const int nrb = (a.N * a.G + 31) / 32, slot = blockIdx.x >> 3;
+    row0 = slot % nrb * 32;
+    c = slot / nrb * 8 + (blockIdx.x & 7);
+    if (c >= a.Hkv * a.nsplit_p) return;
+    h = c / a.nsplit_p;
+    kbeg = (c - h * a.nsplit_p) * a.chunk_p;
+    kend = min(a.P, kbeg + a.chunk_p);
+    n = t0 = 0;
+    step = 1;
+    nrows = a.N * a.G - row0;
+  } else {
+    piece = blockIdx.x - a.n_wave_units;
+    n = (piece >> 2) / a.Hkv;
+    h = (piece >> 2) - n * a.Hkv;
+    t0 = piece & 3;
+    step = 4;
+    row0 = n * a.G;
+    nrows = a.G;
+    kbeg = 0;
+    kend = suffix_len(a, n);
+  }
+  const int ntiles = (kend - kbeg + kTile - 1) / kTile;
+  const int qr = row0 + (r < nrows ? r : 0);
+  V qb[8];
+  load_qt(qb, a.q + ((size_t)(qr / a.G) * a.Hq + h * a.G + qr % a.G) * 128, lane >> 5, r < nrows);
+  RowState st;
+  row_state_init(st);
+  const TileLanes tl = tile_lanes(lane, 0);
+  if constexpr (kPaged != kContig) {
+    const int* table = unit ? a.prefix_pages : a.suffix_pages + (size_t)n * a.max_sp;
+    wave_walk<kWaveStages>(st, qb, smem, smem, tl,
+                           paged_src<kPaged == kPagedNHD>(a, table, unit ? a.P / a.ps : a.max_sp, h, kbeg, kend), kbeg,
+                           t0, ntiles, step, lane);
+  } else {
+    RangeSrc src;
+    src.scale = a.sl2;
+    const size_t off = (unit ? (size_t)h * a.P : ((size_t)n * a.Hkv + h) * a.S) * 128;
+    src.kbase = (unit ? a.kp : a.ks) + off;
+    src.vbase = (unit ? a.vp : a.vs) + off;
+    src.kend = kend;
+    wave_walk<kWaveStages>(st, qb, smem, smem, tl, src, kbeg, t0, ntiles, step, lane);
+  }
+  if (!unit) {
+    if (t0 < ntiles)                                        // the merge does not look past the suffix's tiles
+      store_sums(reinterpret_cast<float*>(a.po_s) + (size_t)piece * a.G * 128, a.pml_s + (size_t)piece * a.G * 2, st,
+                 lane, a.G);
+    return;
+  }
+  const size_t prow = (size_t)c * 32 * a.WRp + row0;        // nrb_p == 1: item c of the row-block layout
+  part_t<elem_t<V>>* po = reinterpret_cast<part_t<elem_t<V>>*>(a.po_p) + prow * 128;
+  static_assert(kWaveStages * kStageBytes >= 32 * 128 * 4, "a unit's ring holds its 32 rows of 128 floats");
+  if (nrows > 16)
+    store_partial_rows_wave<false>(smem, po, a.pml_p + prow * 2, st, lane, nrows);
+  else
+    store_partial<false>(po, a.pml_p + prow * 2, st, lane, nrows);
+}
+
+// The final merge after prefix_waves_kernel: one workgroup per (request, KV head), a wave per row.
+template <class E>
+__global__ __launch_bounds__(256) void prefix_waves_merge_kernel(PrefixArgs a) {
+  typedef part_t<E> PT;
+  __shared__ PT lpo[8 * 128];
+  __shared__ float lpml[8 * 2];
+  const int nh = blockIdx.x, n = nh / a.Hkv, h = nh - n * a.Hkv;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool held = a.G <= 4 && a.nsplit_p <= kPrefetchSplits;
+  PrefixRow pr;
+  if (held && wave < a.G) prefetch_prefix_row<PT>(a, pr, n, h, wave, lane);
+  const int ntiles = (suffix_len(a, n) + kTile - 1) / kTile;
+  for (int gg = wave; gg < a.G; gg += 4) {
+    float2 v[4];
+    float m[4], l[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const size_t row = ((size_t)nh * 4 + u) * a.G + gg;
+      const bool have = u < ntiles;
+      v[u] = have ? *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(a.po_s) + row * 128 + 2 * lane)
+                  : float2{0.f, 0.f};
+      const float2 ml = have ? *reinterpret_cast<const float2*>(a.pml_s + row * 2) : float2{kNegInf, 0.f};
+      m[u] = ml.x;
+      l[u] = ml.y;
+    }
+    const float M = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
+    float lt = 0.f;
+    float2 acc = float2{0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float ak = merge_scale(m[u], M);
+      lt = merge_add(lt, ak, l[u]);
+      acc.x = merge_add(acc.x, ak, v[u].x);
+      acc.y = merge_add(acc.y, ak, v[u].y);
+    }
+    const float inv = part_inv(lt);
+    lpo[gg * 128 + 2 * lane] = (PT)(acc.x * inv);
+    lpo[gg * 128 + 2 * lane + 1] = (PT)(acc.y * inv);
+    if (lane == 0) {
+      lpml[2 * gg] = M;
+      lpml[2 * gg + 1] = lt;
+    }
+  }
+  __syncthreads();
+  if (held) {
+    if (wave < a.G) merge_prefetched_row<E>(a, pr, lpo, lpml, n, h, wave, lane);
+  } else {
+    merge_prefix_rows<E>(a, lpo, lpml, n, h);
+  }
+}
+
 // After a mixed launch with whole suffixes: the final merge of the G rows of (request, KV head), by the functions a
 // fused suffix item uses and from the same partial values, so the output bits do not depend on which path ran.
 template <class E>
@@ -564,6 +695,7 @@ struct PrefixPlan {
   size_t po_p, pml_p, po_s, pml_s, order;
   int n_prefix_items, n_items;
   int units, n_wg_mixed;    // mixed launch: prefix units per workgroup (0: row blocks) and its grid
+  bool waves;               // prefix_waves_kernel instead of the mixed launch
   bool fuse;
 };
 
@@ -611,6 +743,12 @@ static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int
     if ((p.n_prefix_items + 1) / 2 + n_suffix > kDeviceCUs) p.units = 4;
   }
   p.n_wg_mixed = p.units ? (p.n_prefix_items + p.units - 1) / p.units + n_suffix : p.n_items;
+  // More items than the mixed launch runs in one round: single waves (prefix_waves_kernel), up to 96 rows.  us, waves
+  // against the mixed launch (8 KV heads): N = 24, P = 8192 in pages, S <= 1000 30.3 against 33.4; N = 16, P = 16384,
+  // S = 1024 33.7 / 36.4; N = 6 of 8 rows a head, P = 8192 in NHD pages, S <= 500 25.1 / 31.1; N = 13, P = 7409, S = 34
+  // 17.4 / 20.9.  At 128 rows four waves read every prefix tile and the rounds even out: N = 32, P = 4096, S = 256 22.3
+  // / 22.0; N = 32, P = 32768, S = 1000 69.5 / 63.0.  Grids of one round stay mixed: N = 8, P = 2048, S = 256 16.4 / 13.7.
+  p.waves = R <= 96 && p.fuse && G <= 8 && p.n_wg_mixed > kDeviceCUs;
   return p;
 }
 
@@ -649,7 +787,13 @@ static int prefix_launch(PrefixArgs& a, const void* q, void* out, const void* sl
   a.nsplit_s = p.nsplit_s; a.chunk_s = p.chunk_s; a.n_prefix_items = p.n_prefix_items;
   a.sl2 = (float)(1.0 / sqrt((double)D)) * kLog2e;
   prof_before(kKPrefixPartial, s);
-  if (mixed) {
+  if (p.waves) {
+    const int chunks = p.n_prefix_items, nrb = (int)((N * a.G + 31) / 32);   // nrb_p == 1: an item per chunk
+    a.n_wave_units = (chunks + 7) / 8 * 8 * nrb;
+    hipLaunchKernelGGL((prefix_waves_kernel<kPaged, V>), dim3((unsigned)(a.n_wave_units + N * Hkv * 4)), dim3(64), 0, s,
+                       a);
+    VMK_CHECK_HIP(hipGetLastError());
+  } else if (mixed) {
     if (a.mfuse)
       hipLaunchKernelGGL((prefix_mixed_kernel<kPaged, V, true>), dim3((unsigned)p.n_wg_mixed), dim3(256), 0, s, a);
     else
@@ -667,7 +811,12 @@ static int prefix_launch(PrefixArgs& a, const void* q, void* out, const void* sl
     }
   }
   prof_after(kKPrefixPartial, s);
-  if (a.merge) {
+  if (p.waves) {
+    prof_before(kKPrefixCombine, s);
+    hipLaunchKernelGGL(prefix_waves_merge_kernel<elem_t<V>>, dim3((unsigned)(N * Hkv)), dim3(256), 0, s, a);
+    prof_after(kKPrefixCombine, s);
+    VMK_CHECK_HIP(hipGetLastError());
+  } else if (a.merge) {
     prof_before(kKPrefixCombine, s);
     hipLaunchKernelGGL(prefix_merge_kernel<elem_t<V>>, dim3((unsigned)(N * Hkv)), dim3(256), 0, s, a);
     prof_after(kKPrefixCombine, s);
