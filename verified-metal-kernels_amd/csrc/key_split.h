@@ -42,12 +42,13 @@ struct KeySplitArgs {
 // Waves that interleave a split's tiles.
 __host__ __device__ inline int split_waves(int rows) { return rows <= 32 ? 4 : 2; }
 
-// Keys of a split for a group of `rows` query rows in a cache of L positions: 2048 up to 16 rows (decode: 256
-// workgroups once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and longer caches take 4096
-// (32 rows, four requests of 32768 keys: 94 us against 102 with 2048) and, past a million positions, with more than
-// 32 rows, 8192.
+// Keys of a split for a group of `rows` query rows in a cache of L positions: 2048 up to 28 rows (decode: 256
+// workgroups once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and caches past 16384
+// positions take 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919
+// keys: 55.2 us against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows 8192, so that the
+// partials of one group stay within the allocation-free scratch.
 __host__ __device__ inline int split_keys(int rows, int64_t L) {
-  if (rows <= 16 || L <= 16384) return 2048;
+  if (rows <= 16 || L <= (rows <= 28 ? 1 << 20 : 16384)) return 2048;
   return rows > 32 && L > (1 << 20) ? 8192 : 4096;
 }
 
