@@ -157,10 +157,10 @@ struct IkSrc {
 
 // S = iq . ik^T per 32-position tile (M = 64 heads as two 32-row MFMA tiles, N = positions, K = 128 dims), then
 // score = sum_h w[h] * max(S[h], 0) in fp32, and histograms of fkey(score) >> 19 (fine) and >> 24 (coarse) per
-// request.  One item = positions [1024 bx, 1024 bx + 1024) of request b, by NW waves (64 NW threads); each wave
-// streams its 32 / NW tiles through a private NS-stage ring of direct-to-LDS loads; the B operand (ik^T) is read from
+// request.  One item = positions [WG bx, WG bx + WG) of request b, by NW waves (64 NW threads); each wave
+// streams its WG / 32 / NW tiles through a private NS-stage ring of direct-to-LDS loads; the B operand (ik^T) is read from
 // the stage with the attention core's K-operand offsets.  LDS: ring (NW * NS * 8 KB), hist2 (16 KB), chist (1 KB).
-template <class V, int NW, int NS>
+template <class V, int NW, int NS, int WG = kIdxWG>
 __device__ __forceinline__ void indexer_item(const DsaArgs& a, int bx, int b, char* __restrict__ ring,
                                              uint32_t* __restrict__ hist2, uint32_t* __restrict__ chist) {
   static_assert(NS >= 2 && NS <= 4 && NW * 64 >= kCBins && 16 % NW == 0 && NW >= 3,
@@ -203,8 +203,8 @@ __device__ __forceinline__ void indexer_item(const DsaArgs& a, int bx, int b, ch
   src.kbase = a.ik + (size_t)b * a.L * kDI;
   src.vbase = src.kbase;
   src.kend = n;
-  constexpr int kTilesPerWave = kIdxWG / kTile / NW;
-  const int t0 = bx * (kIdxWG / kTile) + wave * kTilesPerWave;   // this wave's first tile
+  constexpr int kTilesPerWave = WG / kTile / NW;
+  const int t0 = bx * (WG / kTile) + wave * kTilesPerWave;   // this wave's first tile
   const int nt = max(0, min(kTilesPerWave, (n + kTile - 1) / kTile - t0));
   const uint32_t ring_off = (uint32_t)wave * NS * kIdxStageBytes;
   const TileLanes tl = tile_lanes(lane, ring_off);
@@ -298,12 +298,14 @@ __device__ __forceinline__ void indexer_item(const DsaArgs& a, int bx, int b, ch
   }
 }
 
-template <class V>
+// WG positions per workgroup: kIdxWG, or kIdxSmallWG (a tile per wave) for calls that would leave most CUs idle.
+constexpr int kIdxSmallWG = kIdxWaves * kTile;
+template <class V, int WG>
 __global__ __launch_bounds__(64 * kIdxWaves) void dsa_indexer_kernel(DsaArgs a) {
   __shared__ __attribute__((aligned(16))) char ring[kIdxWaves * kIdxStages * kIdxStageBytes];
   __shared__ uint32_t hist2[kBins / 2];                     // two 16-bit bin counts per word (<= 1024 per bin)
   __shared__ uint32_t chist[kCBins];
-  indexer_item<V, kIdxWaves, kIdxStages>(a, blockIdx.x, blockIdx.y, ring, hist2, chist);
+  indexer_item<V, kIdxWaves, kIdxStages, WG>(a, blockIdx.x, blockIdx.y, ring, hist2, chist);
 }
 
 // ------------------------------------------------------------------------------------------------ select
@@ -1179,6 +1181,22 @@ static int dsa_fill_args(DsaArgs& a, const void* q, const void* kv, const void* 
   return 0;
 }
 
+// The indexer launch.  Requests of up to 16384 positions that leave three quarters of the CUs idle take smaller
+// workgroups, a tile per wave instead of four in a row.  Whole decode, us, small against large: B = 1, L = 8192 27.1 /
+// 29.9, L = 16000 28.5 / 30.1; B = 8, L = 8192 42.9 / 44.7; B = 4, L = 16384 31.7 / 32.4.  Longer requests lose more by
+// four times as many workgroups adding into one histogram: B = 1, L = 32768 31.0 / 30.5, L = 65536 37.1 / 32.1.
+template <class V>
+static void launch_indexer(const DsaArgs& a, hipStream_t s) {
+  const int64_t wgs = (a.L + kIdxWG - 1) / kIdxWG;
+  if (wgs <= 16 && 4 * wgs * a.B <= kDeviceCUs)
+    hipLaunchKernelGGL((dsa_indexer_kernel<V, kIdxSmallWG>),
+                       dim3((unsigned)((a.L + kIdxSmallWG - 1) / kIdxSmallWG), (unsigned)a.B), dim3(64 * kIdxWaves), 0,
+                       s, a);
+  else
+    hipLaunchKernelGGL((dsa_indexer_kernel<V, kIdxWG>), dim3((unsigned)wgs, (unsigned)a.B), dim3(64 * kIdxWaves), 0, s,
+                       a);
+}
+
 // V: operand type of iq/ik (half8: fp16, bf16x8: bf16); the select works on fp32 scores.
 template <class V>
 static int launch_index_select(const DsaArgs& a, hipStream_t s, bool final_select) {
@@ -1188,8 +1206,7 @@ static int launch_index_select(const DsaArgs& a, hipStream_t s, bool final_selec
       VMK_CHECK_HIP(hipGetLastError());
     }
     prof_before(kKDsaIndexer, s);
-    hipLaunchKernelGGL(dsa_indexer_kernel<V>, dim3((unsigned)((a.L + kIdxWG - 1) / kIdxWG), (unsigned)a.B),
-                       dim3(64 * kIdxWaves), 0, s, a);
+    launch_indexer<V>(a, s);
     prof_after(kKDsaIndexer, s);
     VMK_CHECK_HIP(hipGetLastError());
     prof_before(kKDsaSelectScan, s);
@@ -1276,8 +1293,7 @@ static int dsa_indexer_only(const void* iq, const void* ik, const void* w, const
   a.scores = (float*)scores;
   a.Ls = (int)L;
   a.scores_only = 1;
-  hipLaunchKernelGGL(dsa_indexer_kernel<V>, dim3((unsigned)((L + kIdxWG - 1) / kIdxWG), (unsigned)B),
-                     dim3(64 * kIdxWaves), 0, (hipStream_t)stream, a);
+  launch_indexer<V>(a, (hipStream_t)stream);
   VMK_CHECK_HIP(hipGetLastError());
   return 0;
 }
