@@ -3,23 +3,27 @@
 The key split (decode and verification up to 64 rows per KV head): a call with few splits deals
 units of keys out to all waves and folds them in its combine launch, a call that fills the chip folds them in registers.
 Each case runs a batch large enough for the second and every request alone (the first), which must give the same bits,
-and checks the batch against the float64 oracle.  Sizes: one tile, ends inside the first unit, block and split and just
-past them, fewer tiles than waves, more requests than one scan of the lengths holds, and both row-block forms."""
+and checks the batch against the float64 oracle.  A cache of one split takes one launch without a combine, or units with
+it: the same bits as well.  Sizes: one tile, ends inside the first unit, block and split and just past them, fewer tiles
+than waves, more requests than one scan of the lengths holds, and both row-block forms."""
 import numpy as np
 import pytest
 import torch
 
 import oracle
 from judge import normalised_error as nerr
-from vmk.ops import decode, decode_paged, prefix, prefix_paged, spec
+from vmk.ops import decode, decode_paged, dsa, prefix, prefix_paged, spec
 
 pytestmark = pytest.mark.gpu
 
 DECODE = [dict(B=70, L=40, L_min=1), dict(B=9, L=2049), dict(B=12, L=4096, L_min=1), dict(B=33, L=1025, L_min=1),
-          dict(B=40, L=513, Hq=8, Hkv=1), dict(B=9, L=2500, L_min=1, Hq=64, Hkv=8, dtype="bf16"),
+          dict(B=40, L=513, Hq=8, Hkv=1), dict(B=33, L=1280, L_min=1), dict(B=33, L=1281, L_min=1),
+          dict(B=33, L=2048, L_min=1, dtype="bf16"), dict(B=9, L=2500, L_min=1, Hq=64, Hkv=8, dtype="bf16"),
           dict(B=24, L=6000, L_min=1, Hq=48, Hkv=2)]
-PAGED = [dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16")]
+PAGED = [dict(B=20, L=1504, L_min=1, ps=32, dtype="bf16"), dict(B=20, L=2048, L_min=1, ps=64, layout="NHD"),
+         dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16")]
 SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16), dict(B=9, L=300, k=11, Hq=8, Hkv=2),
+        dict(B=9, L=640, k=16), dict(B=9, L=1500, k=16, dtype="bf16"), dict(B=12, L=2048, k=7),
         dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9)]
 # Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone, which
 # is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows and of fewer
@@ -28,6 +32,9 @@ PREFIX = [dict(N=24, P=8000, S=1000, S_min=0), dict(N=9, P=8191, S=1025, S_min=1
           dict(N=12, P=4100, S=500, S_min=0, Hq=64, dtype="bf16"), dict(N=20, P=5000, S=2048, S_min=1, Hq=16, Hkv=4)]
 PREFIX_PAGED = [dict(N=24, P=8192, S=1000, S_min=0, ps=64, dtype="bf16"),
                 dict(N=11, P=4704, S=700, S_min=0, ps=32, layout="NHD", Hq=64, absent=2)]
+# DSA decode of batches on indexer workgroups of 1024 positions and each request alone on 256: the last workgroup and
+# tile partly filled, one position past the selection, and the longest request that takes the small ones.
+DSA = [dict(B=30, L=2049), dict(B=9, L=8100, dtype="bf16"), dict(B=5, L=16384), dict(B=17, L=4097)]
 
 
 def same_bits(a, b):
@@ -96,3 +103,27 @@ def test_paged_prefix_batch_equals_requests_alone(shape):
     for i in range(shape["N"]):
         assert same_bits(vmk.prefix_decode_paged(**prefix_paged.row_inputs(inp, i))[0], out[i]), i
     check(out, oracle.prefix_paged.ref64(**inp))
+
+
+@pytest.mark.parametrize("shape", DSA)
+def test_dsa_batch_equals_requests_alone(shape):
+    import vmk
+    print(f"dsa {shape}", flush=True)
+    inp = dsa.make_inputs(shape, seed=46, dist="ragged", device="cuda")
+
+    def run(x):
+        B = x["q"].shape[0]
+        idx = torch.full((B, 2048), -1, dtype=torch.int32, device="cuda")
+        cnt = torch.full((B,), -7, dtype=torch.int32, device="cuda")
+        out = vmk.dsa_decode(x["q"], x["kv"], x["iq"], x["ik"], x["w"], x["lens"], idx=idx, cnt=cnt)
+        return out, idx, cnt
+
+    out, idx, cnt = run(inp)
+    scores = vmk.dsa_indexer(inp["iq"], inp["ik"], inp["w"], inp["lens"])
+    for i in range(shape["B"]):
+        x = {k: None if v is None else v[i:i + 1].contiguous() for k, v in inp.items()}
+        o, ix, c = run(x)
+        assert same_bits(o[0], out[i]) and torch.equal(ix[0], idx[i]) and torch.equal(c[0], cnt[i]), i
+        n = int(x["lens"][0])
+        s = vmk.dsa_indexer(x["iq"], x["ik"], x["w"], x["lens"])
+        assert torch.equal(s[0, :n].view(torch.int32), scores[i, :n].view(torch.int32)), i

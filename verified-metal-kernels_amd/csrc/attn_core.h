@@ -16,6 +16,8 @@
 #pragma once
 #include "vmk_common.h"
 
+#include <type_traits>
+
 namespace vmk {
 
 constexpr int kTile = 32;                 // keys per tile
@@ -704,10 +706,16 @@ constexpr int kAttnSmemBytes = 8 * kStageBytes;
 constexpr int kAttnSlotsEnd = 4 * kSlotBytes;
 static_assert(kAttnSlotsEnd <= kAttnSmemBytes, "merge slots must fit in the stage memory");
 
-// kFold: a wave's tiles go in units of `unit` tiles (a power of two), each with a state of its own, folded in order.
-template <int WR, int WK, int NSW = 2, class V = half8, bool kFold = false, class Src, class QRow, class PT>
+// kFold: a wave's tiles go in units of `unit` tiles (a power of two), each with a state of its own, folded in order.  orow(r), when given instead of po, is where row r's result goes, the final output of a split that
+// holds every key of its rows: no (m, l), and a row without any key is NaN (the softmax of no keys is 0 / 0).
+struct NoRow {
+  __device__ __forceinline__ float* operator()(int) const { return nullptr; }
+};
+template <int WR, int WK, int NSW = 2, class V = half8, bool kFold = false, class Src, class QRow, class PT,
+          class ORow = NoRow>
 __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow, int nrows, int kbeg, int ntiles,
-                                          PT* po, float* pml, int unit = 0) {
+                                          PT* po, float* pml, int unit = 0, ORow orow = ORow()) {
+  constexpr bool kFinal = !std::is_same_v<ORow, NoRow>;
   static_assert(WR * WK == 4 && WK > 1 && WR * WK * NSW <= 8, "four waves, rings within the stage memory");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave % WR, wk = wave / WR;
@@ -761,7 +769,7 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
       ltot = merge_add(ltot, ak[k],
                        reinterpret_cast<const float2*>(smem + (k * WR + wr) * kSlotBytes + 64 * 64 * 4)[lane].y);
     }
-    const float inv = part_inv(ltot);
+    const float inv = kFinal ? 1.f / ltot : part_inv(ltot);
 #pragma unroll
     for (int j = 0; j < 4 / WK; ++j) {
       const int dt = wk + j * WK;
@@ -780,9 +788,14 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
       }
       if (r < nvalid)
 #pragma unroll
-        for (int blk = 0; blk < 4; ++blk) store_part4(pob + r * 128 + dt * 32 + 8 * blk + 4 * g, acc[blk] * inv);
+        for (int blk = 0; blk < 4; ++blk) {
+          if constexpr (kFinal)
+            store_part4(orow(row) + dt * 32 + 8 * blk + 4 * g, acc[blk] * inv);
+          else
+            store_part4(pob + r * 128 + dt * 32 + 8 * blk + 4 * g, acc[blk] * inv);
+        }
     }
-    if (wk == 0 && g == 0 && r < nvalid) {
+    if (!kFinal && wk == 0 && g == 0 && r < nvalid) {
       pmlb[2 * r] = M;
       pmlb[2 * r + 1] = ltot;
     }

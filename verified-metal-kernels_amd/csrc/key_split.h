@@ -36,6 +36,7 @@ struct KeySplitArgs {
   int split;               // keys of a split
   int g0, ngrp;            // groups of this launch (with lens: all of them)
   int logw;                // units: log2 of the shares the line of tiles is cut into (four waves each)
+  int one_split;           // L holds one split: it is the result, not weighed and rounded again
   float sl2;               // softmax scale * log2(e)
 };
 
@@ -45,8 +46,8 @@ __host__ __device__ inline int split_waves(int rows) { return rows <= 32 ? 4 : 2
 // Keys of a split for a group of `rows` query rows in a cache of L positions: 2048 up to 28 rows (decode: 256
 // workgroups once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and caches past 16384
 // positions take 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919
-// keys: 55.2 us against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows 8192, so that the
-// partials of one group stay within the allocation-free scratch.
+// keys: 55.2 us against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows
+// 8192, so that the partials of one group stay within the allocation-free scratch.
 __host__ __device__ inline int split_keys(int rows, int64_t L) {
   if (rows <= 16 || L <= (rows <= 28 ? 1 << 20 : 16384)) return 2048;
   return rows > 32 && L > (1 << 20) ? 8192 : 4096;
@@ -412,7 +413,10 @@ struct SplitSrc {
   __device__ void mask(floatx16& s, int key0, int g) const { cm.mask(s, key0, g); }
 };
 
-template <int kSrc, bool kBits, class V>
+// kFinal: a split is a whole group (nsplit == 1); its rows are the result and no combine launch follows.  Rounded once
+// from the fp32 sums, as a split whose combine weighs nothing else.  Decode of one and 16 requests of 1000 keys 15.3 and
+// 16.6 us with the combine, 12.2 and 13.7 without; verification of 16 drafts in four of 2000 keys 35.3 and 32.4.
+template <int kSrc, bool kBits, class V, bool kFinal>
 __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[kAttnSmemBytes];
   const int item = blockIdx.x, grel = item / a.slots, split = item - grel * a.slots;
@@ -427,11 +431,22 @@ __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   typedef part_t<elem_t<V>> PT;
   PT* po = reinterpret_cast<PT*>(a.part_o) + (size_t)item * a.rows_s * 128;
   float* pml = a.part_ml + (size_t)item * a.rows_s * 2;
+  auto orow = [&](int r) {
+    const int i = r / a.G, gg = r - i * a.G;
+    return reinterpret_cast<elem_t<V>*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
+  };
   auto attend = [&](const auto& src) {
+    const auto run = [&](auto WR) {
+      constexpr int kWR = decltype(WR)::value;
+      if constexpr (kFinal)
+        attend_wg<kWR, 4 / kWR, 2, V, true>(smem, src, qrow, R, kbeg, ntiles, po, pml, unit, orow);
+      else
+        attend_wg<kWR, 4 / kWR, 2, V, true>(smem, src, qrow, R, kbeg, ntiles, po, pml, unit);
+    };
     if (kBits && R > 32)                                    // decode with more than 32 rows takes kBits, too
-      attend_wg<2, 2, 2, V, true>(smem, src, qrow, R, kbeg, ntiles, po, pml, unit);
+      run(std::integral_constant<int, 2>());
     else
-      attend_wg<1, 4, 2, V, true>(smem, src, qrow, R, kbeg, ntiles, po, pml, unit);
+      run(std::integral_constant<int, 1>());
   };
   if constexpr (kSrc == kStreamContig) {
     SplitSrc<kBits> src;
@@ -612,6 +627,10 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
     }
   }
   if (tid >= 128) return;
+  if (nsplit == 1 && a.one_split) {                         // the split is the result, as key_split_kernel writes it
+    num = sl[0] == 0.f ? __builtin_nanf("") : (float)so[0][tid];
+    den = 1.f;
+  }
   const int di = row / a.G, gg = row - di * a.G;
   reinterpret_cast<E*>(a.out)[((size_t)(b * a.kd + di) * a.Hq + h * a.G + gg) * 128 + tid] = (E)(num / den);
 }
@@ -631,6 +650,9 @@ struct KeySplitPlan {
 //   keys: 18.5 against 20.2; verification of 8 drafts, 1, 2, 4 requests of 8192 keys: 16.9, 21.3, 40.1 against 30.8,
 //   30.8, 33.4, and 8 of 1000 keys: 20.9 against 16.1; of 16 drafts (64 rows), 1, 2 requests of 32768 keys: 38, 72
 //   against 82, 82, and 8 of 1000 keys: 31.2 against 21.5.
+// A cache of one split of at most ten tiles to a wave is never dealt out: the split alone is one launch.  Decode of one
+// and eight requests of 1000 keys 15.3 and 14.7 us as units, 12.2 and 12.1 as a split; of one of 1500 keys 15.0 and
+// 15.3, of 2048 15.0 and 18.6.
 inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L) {
   KeySplitPlan p;
   p.rows = (int)rows;
@@ -638,7 +660,8 @@ inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L) {
   p.nsplit = (int)((L + p.split - 1) / p.split);
   const int64_t nt = (L + kTile - 1) / kTile;
   p.units = (rows > 32 ? 2 : 4) * ngrp * p.nsplit <= kDeviceCUs && ngrp * rows <= (rows > 32 ? 1024 : 512) &&
-            nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt, p.split);
+            nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt, p.split) &&
+            (p.nsplit > 1 || nt > 10 * split_waves(p.rows));
   p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
   p.rows_s = rows <= 32 || !p.units ? (int)rows : 32;
   p.slots = p.units ? (int)unit_slots((int)rows, nt, p.split) : p.nsplit;
@@ -662,12 +685,18 @@ inline int key_split_launch(KeySplitArgs a, const KeySplitPlan& p, void* partial
   a.part_o = partials;
   a.part_ml = reinterpret_cast<float*>((char*)partials + key_split_ml_offset(p, a.ngrp, sizeof(part_t<E>)));
   a.nrb = p.nrb; a.slots = p.slots; a.rows_s = p.rows_s; a.split = p.split;
+  a.one_split = p.nsplit == 1;
   const int64_t rows = (int64_t)a.ngrp * p.rows;
   if (!p.units) {
     prof_before(kKSpecPartial, s);
-    hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V>), dim3((unsigned)(a.ngrp * p.nsplit)), dim3(256), 0, s, a);
+    if (p.nsplit == 1)
+      hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V, true>), dim3((unsigned)a.ngrp), dim3(256), 0, s, a);
+    else
+      hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V, false>), dim3((unsigned)(a.ngrp * p.nsplit)), dim3(256), 0, s,
+                         a);
     prof_after(kKSpecPartial, s);
     VMK_CHECK_HIP(hipGetLastError());
+    if (p.nsplit == 1) return 0;
     prof_before(kKSpecCombine, s);
     if (rows >= kSplitVecRows)
       hipLaunchKernelGGL(key_split_combine_vec_kernel<E>, dim3((unsigned)((rows + 3) / 4)), dim3(64), 0, s, a);

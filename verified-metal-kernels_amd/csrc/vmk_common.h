@@ -52,6 +52,10 @@ __device__ __forceinline__ void store_part4(float* p, floatx4 v) { *reinterpret_
 __device__ __forceinline__ void store_part4(f16* p, floatx4 v) {
   *reinterpret_cast<half4*>(p) = half4{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
 }
+__device__ __forceinline__ void store_part4(bf16* p, floatx4 v) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
+}
 // The same as non-temporal stores, for partials that are read back only by a later launch: they stream to memory
 // instead of waiting in L2 for the end-of-kernel writeback (C2's prefix partials -2 %; partials that a combine reads
 // right after, as C3's, lose by it).
