@@ -41,8 +41,7 @@ def _drain(key):
 
 def device_ok(device):
     """Raises unless `device` is a ROCm gfx950 device and libvmk.so is loaded (checked once per device)."""
-    idx = torch.device(device).index
-    idx = torch.cuda.current_device() if idx is None else idx
+    idx = _dev_index(device)
     if idx not in _dev_ok:
         if not torch.cuda.is_available():
             raise lib.VmkError("libvmk needs a ROCm GPU; torch.cuda.is_available() is False")
@@ -53,8 +52,9 @@ def device_ok(device):
 
 
 def _dev_index(device):
-    dev = torch.device(device)
-    return dev.index if dev.index is not None else torch.cuda.current_device()
+    if not isinstance(device, torch.device):
+        device = torch.device(device)
+    return device.index if device.index is not None else torch.cuda.current_device()
 
 
 def workspace(nbytes, device):
@@ -109,11 +109,9 @@ def _launch(name, ws, *args):
 
 
 def _stream(t):
-    return ctypes_ptr(torch.cuda.current_stream(t.device).cuda_stream)
-
-
-def ctypes_ptr(x):
-    return int(x)
+    """The handle of the current stream of t's device.  Asked for as a number: torch.cuda.current_stream() builds a
+    Stream object around it on every call (1.8 us of the 13 us that a small decode takes on the host, against 0.1)."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _need(t, name, dtype, ndim):
