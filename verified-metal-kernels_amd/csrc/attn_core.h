@@ -706,8 +706,9 @@ constexpr int kAttnSmemBytes = 8 * kStageBytes;
 constexpr int kAttnSlotsEnd = 4 * kSlotBytes;
 static_assert(kAttnSlotsEnd <= kAttnSmemBytes, "merge slots must fit in the stage memory");
 
-// kFold: a wave's tiles go in units of `unit` tiles (a power of two), each with a state of its own, folded in order.  orow(r), when given instead of po, is where row r's result goes, the final output of a split that
-// holds every key of its rows: no (m, l), and a row without any key is NaN (the softmax of no keys is 0 / 0).
+// kFold: a wave's tiles go in units of `unit` tiles (a power of two), each with a state of its own, folded in order.
+// orow(r), when given instead of po, is where row r's result goes, the final output of a split that holds every key of
+// its rows: no (m, l), and a row without any key is NaN (the softmax of no keys is 0 / 0).
 struct NoRow {
   __device__ __forceinline__ float* operator()(int) const { return nullptr; }
 };

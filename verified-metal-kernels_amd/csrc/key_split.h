@@ -86,7 +86,8 @@ __device__ __forceinline__ int stream_len_uniform(const KeySplitArgs& a, int b) 
 }
 __device__ __forceinline__ int tiles_of(int n) { return (n + kTile - 1) >> 5; }
 
-// A block of split_waves() units' place: its group and first tile within the group; (the first group past the launch's, 0) is the end.
+// A block of split_waves() units' place: its group and first tile within the group; (the first group past the launch's,
+// 0) is the end.
 struct StreamPos {
   int g, t;
 };
