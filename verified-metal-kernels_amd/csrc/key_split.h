@@ -697,7 +697,11 @@ inline int key_split_launch(KeySplitArgs a, const KeySplitPlan& p, void* partial
                          a);
     prof_after(kKSpecPartial, s);
     VMK_CHECK_HIP(hipGetLastError());
-    if (p.nsplit == 1) return 0;
+    if (p.nsplit == 1) {
+      prof_before(kKSpecCombine, s);                        // an armed bracket closes over nothing
+      prof_after(kKSpecCombine, s);
+      return 0;
+    }
     prof_before(kKSpecCombine, s);
     if (rows >= kSplitVecRows)
       hipLaunchKernelGGL(key_split_combine_vec_kernel<E>, dim3((unsigned)((rows + 3) / 4)), dim3(64), 0, s, a);
