@@ -70,7 +70,8 @@ int vmk_spec_verify_noalloc(const void* q, const void* k, const void* v, const v
  *   k, v  (B, Hkv, L, D)   fp16   cache; the token's own key/value is its last position in use
  *   lens  (B,)             int32  positions in use per request (clamped to [1, L]), or NULL: all L
  *   out   (B, Hq, D)       fp16
- * D must be 128, Hq a multiple of Hkv, L >= 1. */
+ * D must be 128, Hq a multiple of Hkv, L >= 1.  A request's output bits depend on its own keys, length and
+ * Hq / Hkv only: not on the other requests, nor on L. */
 size_t vmk_decode_workspace_size(int64_t B, int64_t Hq, int64_t Hkv, int64_t D, int64_t L);
 int vmk_decode(const void* q, const void* k, const void* v, const void* lens, void* out, int64_t B, int64_t Hq,
                int64_t Hkv, int64_t D, int64_t L, void* workspace, size_t ws_bytes, void* stream);

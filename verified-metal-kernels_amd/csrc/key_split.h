@@ -4,8 +4,8 @@
 // four waves (with more than 32 rows, two pairs of waves), and a wave's tiles into units of unit_tiles().  Each unit is
 // walked with a state of its own; a wave's units are folded in order, the waves of a split are merged, the split is
 // rounded to the partial type, and the splits are merged by weight.  This cut, and so a row's arithmetic, is a function
-// of the group's own rows and length only (a request alone gives the same bits as in its batch), while two kinds of
-// launch evaluate it:
+// of the group's own rows and length only (a request gives the same bits alone, in a batch and in a longer cache), while
+// two kinds of launch evaluate it:
 //   * key_split_kernel, one workgroup per split: the units are folded in the waves' registers;
 //   * key_units_kernel, when there are too few splits for the chip (one request of 8192 keys: 32): the units are dealt
 //     out to all waves and stored, and the combine launch folds them (key_units_combine_kernel).
@@ -33,45 +33,55 @@ struct KeySplitArgs {
   int B, kd, Hq, Hkv, G, L, W;
   int ps, max_pages, num_pages;
   int nrb, slots, rows_s;  // row blocks of a group; splits or units per (group, row block), at most; rows of one partial
-  int split;               // keys of a split
   int g0, ngrp;            // groups of this launch (with lens: all of them)
   int logw;                // units: log2 of the shares the line of tiles is cut into (four waves each)
-  int one_split;           // L holds one split: it is the result, not weighed and rounded again
   float sl2;               // softmax scale * log2(e)
 };
 
 // Waves that interleave a split's tiles.
 __host__ __device__ inline int split_waves(int rows) { return rows <= 32 ? 4 : 2; }
 
-// Keys of a split for a group of `rows` query rows in a cache of L positions: 2048 up to 28 rows (decode: 256
-// workgroups once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and caches past 16384
-// positions take 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919
-// keys: 55.2 us against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows
-// 8192, so that the partials of one group stay within the allocation-free scratch.
-__host__ __device__ inline int split_keys(int rows, int64_t L) {
-  if (rows <= 16 || L <= (rows <= 28 ? 1 << 20 : 16384)) return 2048;
-  return rows > 32 && L > (1 << 20) ? 8192 : 4096;
+// Keys of a split for a group of `rows` query rows whose own length is n: 2048 up to 28 rows (decode: 256 workgroups
+// once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and requests past 16384 positions take
+// 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919 keys: 55.2 us
+// against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows 8192, so that
+// the partials of one group stay within the allocation-free scratch.  The steps are whole tiles, so n may be rounded up
+// to its tiles.
+constexpr int64_t kSplitStep1 = 16384, kSplitStep2 = 1 << 20;
+__host__ __device__ inline int split_keys(int rows, int64_t n) {
+  if (rows <= 16 || n <= (rows <= 28 ? kSplitStep2 : kSplitStep1)) return 2048;
+  return rows > 32 && n > kSplitStep2 ? 8192 : 4096;
 }
 
 // Tiles of a unit of a group with nt key tiles: a power of two, about 64 units to a group, at least lo (a unit's
 // partial is rows * 528 bytes, its keys 16 KB a tile), at most the wave's tiles of a split.
-__host__ __device__ inline int unit_tiles(int rows, int nt, int split) {
-  const int lo = rows <= 8 ? 4 : 8, hi = split / (32 * split_waves(rows));
+__host__ __device__ inline int unit_tiles(int rows, int nt) {
+  const int lo = rows <= 8 ? 4 : 8, hi = split_keys(rows, (int64_t)nt * kTile) / (kTile * split_waves(rows));
   int t = lo;
   while (t < hi && 64 * t < nt) t *= 2;
   return t;
 }
 // Units of a group of nt tiles: blocks of split_waves() units, but for a last block of fewer tiles than that.
-__host__ __device__ inline int group_units(int rows, int nt, int split) {
-  const int q = split_waves(rows), bt = q * unit_tiles(rows, nt, split);
+__host__ __device__ inline int group_units(int rows, int nt) {
+  const int q = split_waves(rows), bt = q * unit_tiles(rows, nt);
   const int nb = (nt + bt - 1) / bt, last = nt - (nb - 1) * bt;
   return (nb - 1) * q + (last < q ? last : q);
 }
-// The most that group_units() gives for 1 .. nt tiles (up to 64 units of one size, then of the next; past 64 of the
-// largest size, as many as there are).
-inline int64_t unit_slots(int rows, int64_t nt, int split) {
-  const int64_t q = split_waves(rows), hi = split / 32;
-  return std::max<int64_t>(std::min<int64_t>(64, nt), q * ((nt + hi - 1) / hi));
+// The most splits, and the most units (up to 64 units of one size, then of the next; past 64 of the largest size, as
+// many as there are), of a group of 1 .. L keys.  Both fall where the split size steps up, so the lengths at the steps
+// count, too.
+template <class F>
+inline int64_t most_up_to(int64_t L, F f) {
+  return std::max(f(L), std::max(f(std::min(L, kSplitStep1)), f(std::min(L, kSplitStep2))));
+}
+inline int64_t split_slots(int rows, int64_t L) {
+  return most_up_to(L, [&](int64_t n) { const int64_t s = split_keys(rows, n); return (n + s - 1) / s; });
+}
+inline int64_t unit_slots(int rows, int64_t L) {
+  return most_up_to(L, [&](int64_t n) {
+    const int64_t q = split_waves(rows), nt = (n + kTile - 1) / kTile, hi = split_keys(rows, n) / kTile;
+    return std::max<int64_t>(std::min<int64_t>(64, nt), q * ((nt + hi - 1) / hi));
+  });
 }
 
 // Cache positions of batch entry b: lens[b] clamped to [kd, L] (the query rows are the last kd of them), or L.
@@ -93,8 +103,8 @@ struct StreamPos {
 };
 
 // The first block at or after tile t of group g (nt tiles).
-__device__ __forceinline__ StreamPos stream_snap(int g, int t, int nt, int rows, int split) {
-  const int bt = split_waves(rows) * unit_tiles(rows, nt, split), s = (t + bt - 1) / bt * bt;
+__device__ __forceinline__ StreamPos stream_snap(int g, int t, int nt, int rows) {
+  const int bt = split_waves(rows) * unit_tiles(rows, nt), s = (t + bt - 1) / bt * bt;
   return s >= nt ? StreamPos{g + 1, 0} : StreamPos{g, s};
 }
 
@@ -110,7 +120,7 @@ __device__ __forceinline__ void stream_share(const KeySplitArgs& a, int rows, ui
       const uint64_t x = (total * i) >> a.logw;
       if (x >= total) return StreamPos{a.g0 + a.ngrp, 0};
       const uint64_t g = (x >> 32) ? x / (uint32_t)nt : (uint64_t)((uint32_t)x / (uint32_t)nt);
-      return stream_snap(a.g0 + (int)g, (int)(x - g * (uint32_t)nt), nt, rows, a.split);
+      return stream_snap(a.g0 + (int)g, (int)(x - g * (uint32_t)nt), nt, rows);
     };
     beg = find(w);
     end = find(w + 1);
@@ -143,8 +153,7 @@ __device__ __forceinline__ void stream_share(const KeySplitArgs& a, int rows, ui
         const uint32_t ntb = __builtin_amdgcn_readlane(nt, l);
         const uint64_t rel = x - (run + __builtin_amdgcn_readlane(incl, l) - ntb) * (uint32_t)a.Hkv;
         const uint32_t h = (rel >> 32) ? (uint32_t)(rel / ntb) : (uint32_t)rel / ntb;
-        return stream_snap((64 * c + l) * a.Hkv + (int)h, (int)(rel - (uint64_t)h * ntb), (int)ntb, rows,
-                           a.split);
+        return stream_snap((64 * c + l) * a.Hkv + (int)h, (int)(rel - (uint64_t)h * ntb), (int)ntb, rows);
       }
       run += __builtin_amdgcn_readlane(incl, 63);
     }
@@ -321,7 +330,7 @@ __device__ __forceinline__ void stream_walk(const KeySplitArgs& a, char* __restr
     cm.kend = stream_len_uniform(a, b);
     cm.tail0 = cm.kend - a.kd;
     cnt = tiles_of(cm.kend);
-    bt = q * unit_tiles(R, cnt, a.split);
+    bt = q * unit_tiles(R, cnt);
   };
   enter();
   unit_at();
@@ -414,17 +423,17 @@ struct SplitSrc {
   __device__ void mask(floatx16& s, int key0, int g) const { cm.mask(s, key0, g); }
 };
 
-// kFinal: a split is a whole group (nsplit == 1); its rows are the result and no combine launch follows.  Rounded once
-// from the fp32 sums, as a split whose combine weighs nothing else.  Decode of one and 16 requests of 1000 keys 15.3 and
+// kFinal: no group has more than one split; its rows are the result and no combine launch follows.  (The combines of
+// larger caches write a group's only split as it is, too: the same bits.)  Decode of one and 16 requests of 1000 keys 15.3 and
 // 16.6 us with the combine, 12.2 and 13.7 without; verification of 16 drafts in four of 2000 keys 35.3 and 32.4.
 template <int kSrc, bool kBits, class V, bool kFinal>
 __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[kAttnSmemBytes];
   const int item = blockIdx.x, grel = item / a.slots, split = item - grel * a.slots;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int R = a.kd * a.G, n = stream_len_uniform(a, b), kbeg = split * a.split;
-  const int kend = min(n, kbeg + a.split), ntiles = kbeg < n ? tiles_of(kend - kbeg) : 0;
-  const int unit = unit_tiles(R, tiles_of(n), a.split);
+  const int R = a.kd * a.G, n = stream_len_uniform(a, b), keys = split_keys(R, n), kbeg = split * keys;
+  const int kend = min(n, kbeg + keys), ntiles = kbeg < n ? tiles_of(kend - kbeg) : 0;
+  const int unit = unit_tiles(R, tiles_of(n));
   auto qrow = [&](int r) {
     const int i = r / a.G, gg = r - i * a.G;
     return a.q + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
@@ -471,22 +480,37 @@ __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   }
 }
 
-// The final merge of a row's splits: combine_row's arithmetic (split 0 first) over the splits in use.
+// Splits of a group of n positions.
+__device__ __forceinline__ int group_splits(int rows, int n) {
+  const int s = split_keys(rows, n);
+  return (n + s - 1) / s;
+}
+
+// The final merge of a row's splits: combine_row's arithmetic (split 0 first) over the splits in use.  An only split is
+// the result, rounded once as key_split_kernel writes it where the cache holds no second one (a bf16 row weighed and
+// divided again could round to the other side).
 template <class E>
 __global__ __launch_bounds__(128) void key_split_combine_kernel(KeySplitArgs a) {
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int n = (stream_len_uniform(a, b) + a.split - 1) / a.split;
+  const int n = group_splits(R, stream_len_uniform(a, b));
   const int i = row / a.G, gg = row - i * a.G;
   typedef part_t<E> PT;
+  E* out = reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
+  if (n == 1) {
+    const size_t base = (size_t)grel * a.slots * a.rows_s + row;
+    const float x = (float)reinterpret_cast<const PT*>(a.part_o)[base * 128 + threadIdx.x];
+    out[threadIdx.x] = (E)(a.part_ml[base * 2 + 1] == 0.f ? __builtin_nanf("") : x);
+    return;
+  }
   combine_row<128, 1, PT>(n,
                           [&](int s, const float*& ml, const PT*& o) {
                             const size_t base = ((size_t)grel * a.slots + s) * a.rows_s + row;
                             ml = a.part_ml + base * 2;
                             o = reinterpret_cast<const PT*>(a.part_o) + base * 128;
                           },
-                          reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128);
+                          out);
 }
 
 // The same for many rows (at least kSplitVecRows): one wave per 4 rows, 16 lanes per row, each lane 8 head-dims loaded
@@ -500,16 +524,28 @@ __global__ __launch_bounds__(64) void key_split_combine_vec_kernel(KeySplitArgs 
   if (rowg >= a.ngrp * R) return;                           // a whole row group of lanes
   const int grel = rowg / R, row = rowg - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int n = (stream_len(a, b) + a.split - 1) / a.split;
+  const int n = group_splits(R, stream_len(a, b));
   const int i = row / a.G, gg = row - i * a.G;
   typedef part_t<E> PT;
+  E* out = reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128 + 8 * c;
+  if (n == 1) {
+    const size_t base = (size_t)grel * a.slots * a.rows_s + row;
+    Part8<PT> o;
+    o.load(reinterpret_cast<const PT*>(a.part_o) + base * 128 + 8 * c);
+    const bool none = a.part_ml[base * 2 + 1] == 0.f;
+    float x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = none ? __builtin_nanf("") : o.get(k);
+    store_out8(out, x, 1.f);
+    return;
+  }
   combine_vec<PT>(n,
                   [&](int s, const float*& ml, const PT*& o) {
                     const size_t base = ((size_t)grel * a.slots + s) * a.rows_s + row;
                     ml = a.part_ml + base * 2;
                     o = reinterpret_cast<const PT*>(a.part_o) + base * 128 + 8 * c;
                   },
-                  reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128 + 8 * c);
+                  out);
 }
 
 // One output row per workgroup from stored units: lane group s (16 lanes, eight head-dims each) folds the units of
@@ -524,9 +560,9 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int nt = tiles_of(stream_len_uniform(a, b)), tu = unit_tiles(R, nt, a.split), n = group_units(R, nt, a.split);
-  const int q = split_waves(R), per = a.split / (32 * q * tu);   // waves; units of a wave in a split
-  const int nsplit = (nt * 32 + a.split - 1) / a.split;
+  const int len = stream_len_uniform(a, b), nt = tiles_of(len), tu = unit_tiles(R, nt), n = group_units(R, nt);
+  const int q = split_waves(R), per = split_keys(R, len) / (kTile * q * tu);   // waves; units of a wave in a split
+  const int nsplit = group_splits(R, len);
   const size_t p0 = (((size_t)grel * a.nrb + (row >> 5)) * a.slots) * a.rows_s + (row & 31);
   const float* po = reinterpret_cast<const float*>(a.part_o) + 8 * c;
   auto ml_of = [&](int i) { return *reinterpret_cast<const float2*>(a.part_ml + (p0 + (size_t)i * a.rows_s) * 2); };
@@ -628,7 +664,7 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
     }
   }
   if (tid >= 128) return;
-  if (nsplit == 1 && a.one_split) {                         // the split is the result, as key_split_kernel writes it
+  if (nsplit == 1) {                                        // the split is the result, as key_split_kernel writes it
     num = sl[0] == 0.f ? __builtin_nanf("") : (float)so[0][tid];
     den = 1.f;
   }
@@ -638,7 +674,7 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
 
 // ---- host side
 struct KeySplitPlan {
-  int rows, split, nsplit;
+  int rows, nsplit;        // nsplit: splits of a group of L keys
   bool units;
   int nrb, slots, rows_s;
   size_t grp_rows;         // partial rows of one group
@@ -654,18 +690,20 @@ struct KeySplitPlan {
 // A cache of one split of at most ten tiles to a wave is never dealt out: the split alone is one launch.  Decode of one
 // and eight requests of 1000 keys 15.3 and 14.7 us as units, 12.2 and 12.1 as a split; of one of 1500 keys 15.0 and
 // 15.3, of 2048 15.0 and 18.6.
-inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L) {
+//
+// ragged: a group may be shorter than L (and have more splits than one of L keys, where the split size steps up).
+inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged) {
   KeySplitPlan p;
   p.rows = (int)rows;
-  p.split = split_keys((int)rows, L);
-  p.nsplit = (int)((L + p.split - 1) / p.split);
+  const int split = split_keys((int)rows, L);
+  p.nsplit = (int)((L + split - 1) / split);
   const int64_t nt = (L + kTile - 1) / kTile;
   p.units = (rows > 32 ? 2 : 4) * ngrp * p.nsplit <= kDeviceCUs && ngrp * rows <= (rows > 32 ? 1024 : 512) &&
-            nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt, p.split) &&
+            nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt) &&
             (p.nsplit > 1 || nt > 10 * split_waves(p.rows));
   p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
   p.rows_s = rows <= 32 || !p.units ? (int)rows : 32;
-  p.slots = p.units ? (int)unit_slots((int)rows, nt, p.split) : p.nsplit;
+  p.slots = (int)(p.units ? unit_slots((int)rows, L) : ragged ? split_slots((int)rows, L) : p.nsplit);
   p.grp_rows = (size_t)p.nrb * p.slots * p.rows_s;
   return p;
 }
@@ -685,15 +723,14 @@ inline int key_split_launch(KeySplitArgs a, const KeySplitPlan& p, void* partial
   typedef elem_t<V> E;
   a.part_o = partials;
   a.part_ml = reinterpret_cast<float*>((char*)partials + key_split_ml_offset(p, a.ngrp, sizeof(part_t<E>)));
-  a.nrb = p.nrb; a.slots = p.slots; a.rows_s = p.rows_s; a.split = p.split;
-  a.one_split = p.nsplit == 1;
+  a.nrb = p.nrb; a.slots = p.slots; a.rows_s = p.rows_s;
   const int64_t rows = (int64_t)a.ngrp * p.rows;
   if (!p.units) {
     prof_before(kKSpecPartial, s);
     if (p.nsplit == 1)
       hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V, true>), dim3((unsigned)a.ngrp), dim3(256), 0, s, a);
     else
-      hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V, false>), dim3((unsigned)(a.ngrp * p.nsplit)), dim3(256), 0, s,
+      hipLaunchKernelGGL((key_split_kernel<kSrc, kBits, V, false>), dim3((unsigned)(a.ngrp * p.slots)), dim3(256), 0, s,
                          a);
     prof_after(kKSpecPartial, s);
     VMK_CHECK_HIP(hipGetLastError());
@@ -709,7 +746,7 @@ inline int key_split_launch(KeySplitArgs a, const KeySplitPlan& p, void* partial
       hipLaunchKernelGGL(key_split_combine_kernel<E>, dim3((unsigned)rows), dim3(128), 0, s, a);
   } else {
     const int64_t nt = (a.L + (int64_t)kTile - 1) / kTile;
-    const int64_t bt = split_waves(p.rows) * unit_tiles(p.rows, (int)nt, p.split);
+    const int64_t bt = split_waves(p.rows) * unit_tiles(p.rows, (int)nt);
     const int64_t blocks = (int64_t)a.ngrp * ((nt + bt - 1) / bt);
     // Shares of four waves: a power of two, at least one per block up to four waves on every CU.  Two waves of four
     // stages per workgroup while that leaves CUs free.

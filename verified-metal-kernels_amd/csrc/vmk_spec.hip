@@ -189,7 +189,7 @@ extern "C" size_t vmk_spec_workspace_size(int64_t B, int64_t kd, int64_t Hq, int
   if (B <= 0 || kd <= 0 || Hkv <= 0 || Hq % Hkv || D != 128 || L < kd) return 0;
   const int64_t R = kd * (Hq / Hkv);
   if (!spec_rows_mode(R))
-    return kWsHead + key_split_bytes(key_split_plan(B * Hkv, R, L), B * Hkv, sizeof(float)) + 512;
+    return kWsHead + key_split_bytes(key_split_plan(B * Hkv, R, L, true), B * Hkv, sizeof(float)) + 512;
   SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
   return kWsHead + (p.po_floats + p.pml_floats) * sizeof(float) + 512;   // fits either partial type
 }
@@ -240,7 +240,7 @@ static int spec_call(const void* q, const void* k, const void* v, const void* ma
   a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)G; a.L = (int)L; a.W = (int)W;
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
   const int64_t groups = B * Hkv;
-  const KeySplitPlan p = key_split_plan(groups, R, L);
+  const KeySplitPlan p = key_split_plan(groups, R, L, lens != nullptr);
   int64_t step = groups;
   if (budget)
     step = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(budget / (key_split_bytes(p, 1, sizeof(part_t<elem_t<V>>)) + 256))));
@@ -361,7 +361,7 @@ static int decode_paged(const void* q, const void* k_pages, const void* v_pages,
   a.ps = (int)page_size; a.max_pages = (int)max_pages; a.num_pages = (int)num_pages;
   a.ngrp = (int)(B * Hkv);
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
-  return key_split_launch<kNHD ? kStreamNHD : kStreamHND, false, V>(a, key_split_plan(B * Hkv, a.G, L),
+  return key_split_launch<kNHD ? kStreamNHD : kStreamHND, false, V>(a, key_split_plan(B * Hkv, a.G, L, lens != nullptr),
                                                                     align_up((char*)workspace + kWsHead, 256),
                                                                     (hipStream_t)stream);
 }
