@@ -45,7 +45,9 @@ int vmk_check_device(void);
  *   mask_words (B, kd, W)            uint32  W = ceil(kd/32); bit j%32 of word j/32 of draft i: i may attend draft j
  *                                            (the reference's (B, kd) int32 `bits` is the W = 1 case)
  *   out        (B, kd, Hq, D)        fp16
- * D must be 128, Hq a multiple of Hkv, L >= kd.  Context positions (< L-kd) are visible to every draft. */
+ * D must be 128, Hq a multiple of Hkv, L >= kd.  Context positions (< L-kd) are visible to every draft.
+ * The workspace size (this and decode's, paged or not) never falls as B or L grows: one sized for the largest batch
+ * and cache serves the smaller ones of the same heads and kd. */
 size_t vmk_spec_workspace_size(int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_t D, int64_t L);
 int vmk_spec_verify(const void* q, const void* k, const void* v, const void* mask_words, void* out, int64_t B,
                     int64_t kd, int64_t Hq, int64_t Hkv, int64_t D, int64_t L, int64_t W, void* workspace,

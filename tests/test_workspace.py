@@ -1,6 +1,8 @@
 """The workspace cache of vmk.api on the CPU: allocation, capture state and the device drain are stubbed, so the
 rules themselves are checked without a GPU: geometric growth, outgrown buffers freed unless a graph was captured
 over them, growth refused during capture, and a failed call setting its buffer aside only after a launch error."""
+import os
+
 import pytest
 import torch
 
@@ -81,3 +83,32 @@ def test_error_codes_are_kept():
     e = lib.VmkError("x", code=2)
     assert e.code == lib.LAUNCH_ERROR and isinstance(e, RuntimeError)
     assert lib.VmkError("y").code is None
+
+
+@pytest.mark.parametrize("op,heads", [("decode", (32, 8)), ("decode", (16, 1)), ("decode", (96, 4)), ("decode", (64, 1)),
+                                      ("paged", (32, 8)), ("paged", (8, 1)),
+                                      (2, (32, 8)), (7, (32, 8)), (8, (32, 8)), (9, (32, 8)), (16, (32, 8)), (16, (4, 1)),
+                                      (64, (32, 8))])
+def test_sizes_grow_with_the_batch_and_the_cache(op, heads):
+    """A workspace sized for the largest batch and cache serves every smaller call: the sizes never fall as either
+    grows.  Sizes around tiles, splits and the lengths at which the split size steps up."""
+    if not os.path.exists(lib.LIB_PATH):
+        pytest.skip("libvmk.so not built")
+    so = lib.load()
+
+    def size(B, L):
+        if op == "decode":
+            return so.vmk_decode_workspace_size(B, *heads, 128, L)
+        if op == "paged":
+            return so.vmk_decode_paged_workspace_size(B, *heads, 128, 32, -(-L // 32))
+        return so.vmk_spec_workspace_size(B, op, *heads, 128, L)
+    batches = [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 128, 300]
+    lengths = sorted({max(64, base + d) for base in (64, 100, 1024, 2048, 4096, 8192, 16384, 20480, 32768, 40960, 65536,
+                                                     131072, 262144, 1 << 20) for d in (-1, 0, 1, 33)})
+    table = [[size(B, n) for n in lengths] for B in batches]
+    assert all(v > 0 for row in table for v in row)
+    for i, row in enumerate(table):
+        for j in range(1, len(row)):
+            assert row[j] >= row[j - 1], (batches[i], lengths[j - 1], lengths[j])
+        if i:
+            assert all(a >= b for a, b in zip(row, table[i - 1])), (batches[i - 1], batches[i])

@@ -680,6 +680,10 @@ struct KeySplitPlan {
   size_t grp_rows;         // partial rows of one group
 };
 
+// The most splits and rows of a unit launch.
+inline int64_t unit_max_splits(int rows) { return kDeviceCUs / (rows > 32 ? 2 : 4); }
+inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
+
 // Units while the splits of all groups (at their longest) leave three quarters of the CUs without one (half, with more
 // than 32 rows, whose tiles cost two waves), there are units to deal out, and the rows are few enough that the units'
 // stores and their merge do not cost more than the wider walk saves.  Measured, us, units against splits:
@@ -698,7 +702,7 @@ inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool r
   const int split = split_keys((int)rows, L);
   p.nsplit = (int)((L + split - 1) / split);
   const int64_t nt = (L + kTile - 1) / kTile;
-  p.units = (rows > 32 ? 2 : 4) * ngrp * p.nsplit <= kDeviceCUs && ngrp * rows <= (rows > 32 ? 1024 : 512) &&
+  p.units = ngrp * p.nsplit <= unit_max_splits(p.rows) && ngrp * rows <= unit_max_rows(p.rows) &&
             nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt) &&
             (p.nsplit > 1 || nt > 10 * split_waves(p.rows));
   p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
@@ -714,6 +718,20 @@ inline size_t key_split_ml_offset(const KeySplitPlan& p, int64_t ngrp, size_t e)
 }
 inline size_t key_split_bytes(const KeySplitPlan& p, int64_t ngrp, size_t e) {
   return key_split_ml_offset(p, ngrp, e) + ngrp * p.grp_rows * 2 * sizeof(float);
+}
+
+// Bytes of partials, in fp32, that hold those of any call of up to ngrp groups over caches of up to L positions, so that
+// one workspace sized for the largest call serves the smaller ones: a call of fewer groups may take units, which need
+// more than the splits of many groups do.  A unit launch has at most unit_max_splits() splits and unit_max_rows() rows,
+// and a group at most 64 units or split_waves() to a split.
+inline size_t key_split_max_bytes(int64_t ngrp, int64_t rows64, int64_t L) {
+  const int rows = (int)rows64, q = split_waves(rows);
+  const int64_t cap = std::min(ngrp, std::min(unit_max_splits(rows), unit_max_rows(rows) / rows));
+  const int64_t units = std::max(cap * std::min<int64_t>(64, (L + kTile - 1) / kTile),
+                                 q * std::min(unit_max_splits(rows), ngrp * split_slots(rows, L)));
+  const size_t unit_rows = (size_t)units * ((rows + 31) / 32) * (rows <= 32 ? rows : 32);
+  const size_t split_rows = (size_t)ngrp * split_slots(rows, L) * rows;
+  return std::max(unit_rows, split_rows) * (128 + 2) * sizeof(float) + 256;
 }
 
 // Partial and combine launches over the groups [a.g0, a.g0 + a.ngrp), partials at `partials`

@@ -189,7 +189,7 @@ extern "C" size_t vmk_spec_workspace_size(int64_t B, int64_t kd, int64_t Hq, int
   if (B <= 0 || kd <= 0 || Hkv <= 0 || Hq % Hkv || D != 128 || L < kd) return 0;
   const int64_t R = kd * (Hq / Hkv);
   if (!spec_rows_mode(R))
-    return kWsHead + key_split_bytes(key_split_plan(B * Hkv, R, L, true), B * Hkv, sizeof(float)) + 512;
+    return kWsHead + key_split_max_bytes(B * Hkv, R, L) + 512;
   SpecPlan p = spec_plan(B, kd, Hq, Hkv, L);
   return kWsHead + (p.po_floats + p.pml_floats) * sizeof(float) + 512;   // fits either partial type
 }
