@@ -63,3 +63,40 @@ def test_noalloc_on_a_side_stream():
         vmk.spec_verify_noalloc(inp["q"], inp["k"], inp["v"], words, out)
     torch.cuda.synchronize()
     assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
+def launches(call):
+    """Launches of one call, as nodes of its HIP graph."""
+    import ctypes
+    import glob
+    import os
+    path = glob.glob(os.path.join(os.path.dirname(torch.__file__), "lib", "libamdhip64.so*"))[0]   # the one in use
+    hip = ctypes.CDLL(path)
+    call()                                             # what is looked up once is looked up before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    n = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("shape,want_launches", [
+    (dict(B=2, L=8192, k=16), 2),         # as units its partials would not fit: splits, not steps of units
+    (dict(B=4, L=3000, k=9, Hkv=4, Hq=16), 2),
+    (dict(B=1, L=8192, k=16), 2),         # units that fit
+    (dict(B=32, L=16384, k=16), 4),       # the splits of 256 KV heads take two steps
+    (dict(B=41, L=16000, k=14), 4),
+])
+def test_noalloc_in_few_even_launches(shape, want_launches):
+    """Calls whose unit partials exceed the scratch run as splits, and calls whose split partials do run in as few
+    steps as hold them, with the bits of the workspace entry point."""
+    print(f"noalloc launches {shape}", flush=True)
+    inp = spec.make_inputs(shape, seed=5, dist="randn", device="cuda")
+    out = torch.full_like(inp["q"], float("nan"))
+    call_noalloc(inp, out)
+    want = call_workspace(inp)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+    assert launches(lambda: call_noalloc(inp, out)) == want_launches

@@ -680,6 +680,14 @@ struct KeySplitPlan {
   size_t grp_rows;         // partial rows of one group
 };
 
+// Bytes of the O rows (to the next 256-byte boundary) and of all partials of ngrp groups; e: bytes of a split's element.
+inline size_t key_split_ml_offset(const KeySplitPlan& p, int64_t ngrp, size_t e) {
+  return (ngrp * p.grp_rows * 128 * (p.units ? sizeof(float) : e) + 255) / 256 * 256;
+}
+inline size_t key_split_bytes(const KeySplitPlan& p, int64_t ngrp, size_t e) {
+  return key_split_ml_offset(p, ngrp, e) + ngrp * p.grp_rows * 2 * sizeof(float);
+}
+
 // The most splits and rows of a unit launch.
 inline int64_t unit_max_splits(int rows) { return kDeviceCUs / (rows > 32 ? 2 : 4); }
 inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
@@ -696,7 +704,9 @@ inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
 // 15.3, of 2048 15.0 and 18.6.
 //
 // ragged: a group may be shorter than L (and have more splits than one of L keys, where the split size steps up).
-inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged) {
+// room: bytes there are for the partials of all groups (a split's element takes e); units that need more stay splits,
+// with the same bits.
+inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged, size_t e, size_t room) {
   KeySplitPlan p;
   p.rows = (int)rows;
   const int split = split_keys((int)rows, L);
@@ -705,19 +715,18 @@ inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool r
   p.units = ngrp * p.nsplit <= unit_max_splits(p.rows) && ngrp * rows <= unit_max_rows(p.rows) &&
             nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt) &&
             (p.nsplit > 1 || nt > 10 * split_waves(p.rows));
-  p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
-  p.rows_s = rows <= 32 || !p.units ? (int)rows : 32;
-  p.slots = (int)(p.units ? unit_slots((int)rows, L) : ragged ? split_slots((int)rows, L) : p.nsplit);
-  p.grp_rows = (size_t)p.nrb * p.slots * p.rows_s;
+  auto lay_out = [&] {
+    p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
+    p.rows_s = rows <= 32 || !p.units ? (int)rows : 32;
+    p.slots = (int)(p.units ? unit_slots((int)rows, L) : ragged ? split_slots((int)rows, L) : p.nsplit);
+    p.grp_rows = (size_t)p.nrb * p.slots * p.rows_s;
+  };
+  lay_out();
+  if (p.units && key_split_bytes(p, ngrp, e) > room) {
+    p.units = false;
+    lay_out();
+  }
   return p;
-}
-
-// Bytes of the O rows (to the next 256-byte boundary) and of all partials of ngrp groups; e: bytes of a split's element.
-inline size_t key_split_ml_offset(const KeySplitPlan& p, int64_t ngrp, size_t e) {
-  return (ngrp * p.grp_rows * 128 * (p.units ? sizeof(float) : e) + 255) / 256 * 256;
-}
-inline size_t key_split_bytes(const KeySplitPlan& p, int64_t ngrp, size_t e) {
-  return key_split_ml_offset(p, ngrp, e) + ngrp * p.grp_rows * 2 * sizeof(float);
 }
 
 // Bytes of partials, in fp32, that hold those of any call of up to ngrp groups over caches of up to L positions, so that

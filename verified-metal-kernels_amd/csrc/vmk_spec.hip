@@ -218,12 +218,12 @@ static int spec_rows_launch(SpecArgs& a, const SpecPlan& p, void* partials, hipS
 }
 
 // One spec or decode call over contiguous caches, key split or row split by its rows per KV head.  Partials go to
-// `partials` (256-byte aligned); budget: with more groups than its bytes hold partials for, the key split goes through
-// the groups in several launches (0: no limit).
+// `partials` (256-byte aligned, `room` bytes).  Where those hold fewer groups' splits than the call has (the
+// allocation-free scratch; a workspace never does), the key split goes through the groups in equal steps.
 template <class V>
 static int spec_call(const void* q, const void* k, const void* v, const void* mask_words, const void* lens, void* out,
                      int64_t B, int64_t kd, int64_t Hq, int64_t Hkv, int64_t L, int64_t W, void* partials,
-                     size_t budget, hipStream_t s) {
+                     size_t room, hipStream_t s) {
   const int64_t G = Hq / Hkv, R = kd * G;
   if (spec_rows_mode(R)) {
     SpecArgs a;
@@ -240,10 +240,14 @@ static int spec_call(const void* q, const void* k, const void* v, const void* ma
   a.B = (int)B; a.kd = (int)kd; a.Hq = (int)Hq; a.Hkv = (int)Hkv; a.G = (int)G; a.L = (int)L; a.W = (int)W;
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
   const int64_t groups = B * Hkv;
-  const KeySplitPlan p = key_split_plan(groups, R, L, lens != nullptr);
-  int64_t step = groups;
-  if (budget)
-    step = std::min<int64_t>(groups, std::max<int64_t>(1, (int64_t)(budget / (key_split_bytes(p, 1, sizeof(part_t<elem_t<V>>)) + 256))));
+  constexpr size_t e = sizeof(part_t<elem_t<V>>);
+  const KeySplitPlan p = key_split_plan(groups, R, L, lens != nullptr, e, room);
+  int64_t steps = 1, step = groups;
+  while (key_split_bytes(p, step, e) > room) {
+    VMK_CHECK(step > 1, "no room for the partials of one KV head");
+    step = (groups + steps) / (steps + 1);
+    ++steps;
+  }
   for (int64_t g0 = 0; g0 < groups; g0 += step) {
     a.g0 = (int)g0;
     a.ngrp = (int)std::min(step, groups - g0);
@@ -276,8 +280,9 @@ static int spec_verify(const void* q, const void* k, const void* v, const void* 
   if (int rc = spec_check_args(q, k, v, mask_words, out, B, kd, Hq, Hkv, D, L, W)) return rc;
   const size_t need = vmk_spec_workspace_size(B, kd, Hq, Hkv, D, L);
   VMK_CHECK(workspace && ws_bytes >= need, "workspace too small (query vmk_spec_workspace_size)");
-  return spec_call<V>(q, k, v, mask_words, nullptr, out, B, kd, Hq, Hkv, L, W,
-                      align_up((char*)workspace + kWsHead, 256), 0, (hipStream_t)stream);
+  char* partials = (char*)align_up((char*)workspace + kWsHead, 256);
+  return spec_call<V>(q, k, v, mask_words, nullptr, out, B, kd, Hq, Hkv, L, W, partials,
+                      (char*)workspace + ws_bytes - partials, (hipStream_t)stream);
 }
 
 // Plain single-token decode: the verify path with one query row per request and no mask (the row's own position is
@@ -297,8 +302,9 @@ static int decode(const void* q, const void* k, const void* v, const void* lens,
   VMK_CHECK(aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out), "tensors must be 16-byte aligned");
   const size_t need = vmk_decode_workspace_size(B, Hq, Hkv, D, L);
   VMK_CHECK(workspace && ws_bytes >= need, "workspace too small (query vmk_decode_workspace_size)");
-  return spec_call<V>(q, k, v, nullptr, lens, out, B, 1, Hq, Hkv, L, 1, align_up((char*)workspace + kWsHead, 256), 0,
-                      (hipStream_t)stream);
+  char* partials = (char*)align_up((char*)workspace + kWsHead, 256);
+  return spec_call<V>(q, k, v, nullptr, lens, out, B, 1, Hq, Hkv, L, 1, partials,
+                      (char*)workspace + ws_bytes - partials, (hipStream_t)stream);
 }
 
 extern "C" int vmk_spec_verify(const void* q, const void* k, const void* v, const void* mask_words, void* out,
@@ -361,9 +367,10 @@ static int decode_paged(const void* q, const void* k_pages, const void* v_pages,
   a.ps = (int)page_size; a.max_pages = (int)max_pages; a.num_pages = (int)num_pages;
   a.ngrp = (int)(B * Hkv);
   a.sl2 = (float)(1.0 / sqrt(128.0)) * kLog2e;
-  return key_split_launch<kNHD ? kStreamNHD : kStreamHND, false, V>(a, key_split_plan(B * Hkv, a.G, L, lens != nullptr),
-                                                                    align_up((char*)workspace + kWsHead, 256),
-                                                                    (hipStream_t)stream);
+  char* partials = (char*)align_up((char*)workspace + kWsHead, 256);
+  const KeySplitPlan p = key_split_plan(B * Hkv, a.G, L, lens != nullptr, sizeof(part_t<elem_t<V>>),
+                                        (char*)workspace + ws_bytes - partials);
+  return key_split_launch<kNHD ? kStreamNHD : kStreamHND, false, V>(a, p, partials, (hipStream_t)stream);
 }
 
 #define VMK_DECODE_PAGED_ENTRY(name, nhd, V)                                                                      \
