@@ -426,10 +426,23 @@ struct SplitSrc {
 // kFinal: no group has more than one split; its rows are the result and no combine launch follows.  (The combines of
 // larger caches write a group's only split as it is, too: the same bits.)  Decode of one and 16 requests of 1000 keys 15.3 and
 // 16.6 us with the combine, 12.2 and 13.7 without; verification of 16 drafts in four of 2000 keys 35.3 and 32.4.
+//
+// Ragged lengths: workgroup id i runs on XCD i modulo 8, so with eight splits to a group (16384 positions) split 7 of
+// every group, which only the longest requests have, would run on one XCD and split 0, which all have, on another.  The
+// splits of each next group that starts on the same XCD are therefore rotated by one.  Lengths of 1/16 to all of the
+// cache, us, without and with: 4 rows, 8 requests in 16384 positions 63.6 and 46.9; 24 rows (4 KV heads), 64 requests
+// 266 and 213; 32 rows (2 KV heads), 32 requests 69.3 and 57.6.  Split-major order balances as well, but leaves the
+// workgroups without keys for the end: 8 requests in 32768 positions 126 against 119.
 template <int kSrc, bool kBits, class V, bool kFinal>
 __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   __shared__ __attribute__((aligned(16))) char smem[kAttnSmemBytes];
-  const int item = blockIdx.x, grel = item / a.slots, split = item - grel * a.slots;
+  const int grel = blockIdx.x / a.slots;
+  int split = blockIdx.x - grel * a.slots;
+  if (a.lens) {
+    split += (grel >> (3 - min(3, __builtin_ctz(a.slots)))) % a.slots;
+    if (split >= a.slots) split -= a.slots;
+  }
+  const int item = grel * a.slots + split;                  // where the partial goes
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
   const int R = a.kd * a.G, n = stream_len_uniform(a, b), keys = split_keys(R, n), kbeg = split * keys;
   const int kend = min(n, kbeg + keys), ntiles = kbeg < n ? tiles_of(kend - kbeg) : 0;
