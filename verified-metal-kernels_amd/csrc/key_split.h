@@ -1,11 +1,11 @@
 // Key split of attention over few query rows per KV head (decode, chain verification: up to 64 rows).
 //
-// The keys of a group (request, KV head) are cut into splits of split_keys(), a split's tiles are dealt round robin to
-// four waves (with more than 32 rows, two pairs of waves), and a wave's tiles into units of unit_tiles().  Each unit is
-// walked with a state of its own; a wave's units are folded in order, the waves of a split are merged, the split is
-// rounded to the partial type, and the splits are merged by weight.  This cut, and so a row's arithmetic, is a function
-// of the group's own rows and length only (a request gives the same bits alone, in a batch and in a longer cache), while
-// two kinds of launch evaluate it:
+// The keys of a group (request, KV head) are cut into splits of 2048 to 8192 (split_log2()), a split's tiles are dealt
+// round robin to four waves (with more than 32 rows, two pairs of waves), and a wave's tiles into units (unit_log2()).
+// Each unit is walked with a state of its own; a wave's units are folded in order, the waves of a split are merged, the
+// split is rounded to the partial type, and the splits are merged by weight.  This cut, and so a row's arithmetic, is a
+// function of the group's own rows and length only (a request gives the same bits alone, in a batch and in a longer
+// cache), while two kinds of launch evaluate it:
 //   * key_split_kernel, one workgroup per split: the units are folded in the waves' registers;
 //   * key_units_kernel, when there are too few splits for the chip (one request of 8192 keys: 32): the units are dealt
 //     out to all waves and stored, and the combine launch folds them (key_units_combine_kernel).
@@ -40,31 +40,40 @@ struct KeySplitArgs {
 
 // Waves that interleave a split's tiles.
 __host__ __device__ inline int split_waves(int rows) { return rows <= 32 ? 4 : 2; }
+__host__ __device__ inline int split_waves_log2(int rows) { return rows <= 32 ? 2 : 1; }
 
-// Keys of a split for a group of `rows` query rows whose own length is n: 2048 up to 28 rows (decode: 256 workgroups
-// once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and requests past 16384 positions take
-// 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919 keys: 55.2 us
-// against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows 8192, so that
-// the partials of one group stay within the allocation-free scratch.  The steps are whole tiles, so n may be rounded up
-// to its tiles.
-constexpr int64_t kSplitStep1 = 16384, kSplitStep2 = 1 << 20;
-__host__ __device__ inline int split_keys(int rows, int64_t n) {
-  if (rows <= 16 || n <= (rows <= 28 ? kSplitStep2 : kSplitStep1)) return 2048;
-  return rows > 32 && n > kSplitStep2 ? 8192 : 4096;
+// log2 of the keys of a split, for a group of `rows` query rows whose own length is n: 2048 keys up to 28 rows (decode:
+// 256 workgroups once B * Hkv * L reaches 2^19).  With more rows a split's partial is larger, and requests past 16384
+// positions take 4096 (32 rows, four requests of 32768 keys: 94 us against 102 with 2048; 24 rows, one request of 50919
+// keys: 55.2 us against 46.8); past a million positions every split of more than 16 rows does, and of more than 32 rows
+// 8192, so that the partials of one group stay within the allocation-free scratch.  The steps are whole tiles, so n may
+// be rounded up to its tiles.  Shifts: divisions made one request of 8 drafts over 8192 keys 0.25 us longer.
+constexpr int kSplitStep1 = 16384, kSplitStep2 = 1 << 20;
+template <class N>
+__host__ __device__ inline int split_log2(int rows, N n) {
+  if (rows <= 16 || n <= (rows <= 28 ? kSplitStep2 : kSplitStep1)) return 11;
+  return rows > 32 && n > kSplitStep2 ? 13 : 12;
+}
+// Splits of a group of n positions.
+template <class N>
+__host__ __device__ inline N group_splits(int rows, N n) {
+  const int s = split_log2(rows, n);
+  return (n + (1 << s) - 1) >> s;
 }
 
-// Tiles of a unit of a group with nt key tiles: a power of two, about 64 units to a group, at least lo (a unit's
-// partial is rows * 528 bytes, its keys 16 KB a tile), at most the wave's tiles of a split.
-__host__ __device__ inline int unit_tiles(int rows, int nt) {
-  const int lo = rows <= 8 ? 4 : 8, hi = split_keys(rows, (int64_t)nt * kTile) / (kTile * split_waves(rows));
-  int t = lo;
-  while (t < hi && 64 * t < nt) t *= 2;
+// log2 of the tiles of a unit of a group with nt key tiles: about 64 units to a group, at least four or eight tiles (a
+// unit's partial is rows * 528 bytes, its keys 16 KB a tile), at most the wave's tiles of a split.
+__host__ __device__ inline int unit_log2(int rows, int nt) {
+  const int hi = split_log2(rows, nt * kTile) - 5 - split_waves_log2(rows);
+  int t = rows <= 8 ? 2 : 3;
+  while (t < hi && (64 << t) < nt) ++t;
   return t;
 }
+__host__ __device__ inline int unit_tiles(int rows, int nt) { return 1 << unit_log2(rows, nt); }
 // Units of a group of nt tiles: blocks of split_waves() units, but for a last block of fewer tiles than that.
 __host__ __device__ inline int group_units(int rows, int nt) {
-  const int q = split_waves(rows), bt = q * unit_tiles(rows, nt);
-  const int nb = (nt + bt - 1) / bt, last = nt - (nb - 1) * bt;
+  const int q = split_waves(rows), bt = unit_log2(rows, nt) + split_waves_log2(rows);   // tiles of a block, log2
+  const int nb = (nt + (1 << bt) - 1) >> bt, last = nt - ((nb - 1) << bt);
   return (nb - 1) * q + (last < q ? last : q);
 }
 // The most splits, and the most units (up to 64 units of one size, then of the next; past 64 of the largest size, as
@@ -72,15 +81,14 @@ __host__ __device__ inline int group_units(int rows, int nt) {
 // count, too.
 template <class F>
 inline int64_t most_up_to(int64_t L, F f) {
-  return std::max(f(L), std::max(f(std::min(L, kSplitStep1)), f(std::min(L, kSplitStep2))));
+  return std::max(f(L), std::max(f(std::min<int64_t>(L, kSplitStep1)), f(std::min<int64_t>(L, kSplitStep2))));
 }
 inline int64_t split_slots(int rows, int64_t L) {
-  return most_up_to(L, [&](int64_t n) { const int64_t s = split_keys(rows, n); return (n + s - 1) / s; });
+  return most_up_to(L, [&](int64_t n) { return group_splits(rows, n); });
 }
 inline int64_t unit_slots(int rows, int64_t L) {
   return most_up_to(L, [&](int64_t n) {
-    const int64_t q = split_waves(rows), nt = (n + kTile - 1) / kTile, hi = split_keys(rows, n) / kTile;
-    return std::max<int64_t>(std::min<int64_t>(64, nt), q * ((nt + hi - 1) / hi));
+    return std::max<int64_t>(std::min<int64_t>(64, (n + kTile - 1) / kTile), split_waves(rows) * group_splits(rows, n));
   });
 }
 
@@ -104,7 +112,7 @@ struct StreamPos {
 
 // The first block at or after tile t of group g (nt tiles).
 __device__ __forceinline__ StreamPos stream_snap(int g, int t, int nt, int rows) {
-  const int bt = split_waves(rows) * unit_tiles(rows, nt), s = (t + bt - 1) / bt * bt;
+  const int bt = unit_log2(rows, nt) + split_waves_log2(rows), s = ((t + (1 << bt) - 1) >> bt) << bt;
   return s >= nt ? StreamPos{g + 1, 0} : StreamPos{g, s};
 }
 
@@ -317,11 +325,11 @@ __device__ __forceinline__ void stream_walk(const KeySplitArgs& a, char* __restr
   V qb[8];
   StreamMask<kBits> cm;
   cm.scale = a.sl2;
-  int cg = dma.g, ct = dma.t, cnt, unit, uend, bt;
+  int cg = dma.g, ct = dma.t, cnt, unit, uend, bt;         // bt: tiles of a block, log2
   auto unit_at = [&]() {                                    // the unit of tile ct, and the first tile past its block
-    const int blk = ct / bt;
+    const int blk = ct >> bt;
     unit = blk * q + u;
-    uend = min(cnt, (blk + 1) * bt);
+    uend = min(cnt, (blk + 1) << bt);
   };
   auto enter = [&]() {                                      // the compute cursor enters group cg at tile ct
     const int b = cg / a.Hkv, h = cg - b * a.Hkv;
@@ -330,7 +338,7 @@ __device__ __forceinline__ void stream_walk(const KeySplitArgs& a, char* __restr
     cm.kend = stream_len_uniform(a, b);
     cm.tail0 = cm.kend - a.kd;
     cnt = tiles_of(cm.kend);
-    bt = q * unit_tiles(R, cnt);
+    bt = unit_log2(R, cnt) + split_waves_log2(R);
   };
   enter();
   unit_at();
@@ -444,8 +452,8 @@ __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
   }
   const int item = grel * a.slots + split;                  // where the partial goes
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int R = a.kd * a.G, n = stream_len_uniform(a, b), keys = split_keys(R, n), kbeg = split * keys;
-  const int kend = min(n, kbeg + keys), ntiles = kbeg < n ? tiles_of(kend - kbeg) : 0;
+  const int R = a.kd * a.G, n = stream_len_uniform(a, b), keys = split_log2(R, n), kbeg = split << keys;
+  const int kend = min(n, kbeg + (1 << keys)), ntiles = kbeg < n ? tiles_of(kend - kbeg) : 0;
   const int unit = unit_tiles(R, tiles_of(n));
   auto qrow = [&](int r) {
     const int i = r / a.G, gg = r - i * a.G;
@@ -491,12 +499,6 @@ __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
     attend(paged_src<kSrc == kStreamNHD>(a.k, a.v, a.ps, a.Hkv, a.num_pages, a.sl2,
                                          a.pages + (size_t)b * a.max_pages, a.max_pages, h, kbeg, kend));
   }
-}
-
-// Splits of a group of n positions.
-__device__ __forceinline__ int group_splits(int rows, int n) {
-  const int s = split_keys(rows, n);
-  return (n + s - 1) / s;
 }
 
 // The final merge of a row's splits: combine_row's arithmetic (split 0 first) over the splits in use.  An only split is
@@ -573,8 +575,8 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int len = stream_len_uniform(a, b), nt = tiles_of(len), tu = unit_tiles(R, nt), n = group_units(R, nt);
-  const int q = split_waves(R), per = split_keys(R, len) / (kTile * q * tu);   // waves; units of a wave in a split
+  const int len = stream_len_uniform(a, b), nt = tiles_of(len), n = group_units(R, nt), q = split_waves(R);   // q: waves of a split
+  const int per = 1 << (split_log2(R, len) - 5 - split_waves_log2(R) - unit_log2(R, nt));   // units of a wave in a split
   const int nsplit = group_splits(R, len);
   const size_t p0 = (((size_t)grel * a.nrb + (row >> 5)) * a.slots) * a.rows_s + (row & 31);
   const float* po = reinterpret_cast<const float*>(a.part_o) + 8 * c;
@@ -722,8 +724,7 @@ inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
 inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged, size_t e, size_t room) {
   KeySplitPlan p;
   p.rows = (int)rows;
-  const int split = split_keys((int)rows, L);
-  p.nsplit = (int)((L + split - 1) / split);
+  p.nsplit = (int)group_splits((int)rows, L);
   const int64_t nt = (L + kTile - 1) / kTile;
   p.units = ngrp * p.nsplit <= unit_max_splits(p.rows) && ngrp * rows <= unit_max_rows(p.rows) &&
             nt > split_waves(p.rows) * unit_tiles(p.rows, (int)nt) &&
