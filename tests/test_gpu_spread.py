@@ -26,12 +26,16 @@ SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16)
         dict(B=9, L=640, k=16), dict(B=9, L=1500, k=16, dtype="bf16"), dict(B=12, L=2048, k=7),
         dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9)]
 # Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone, which
-# is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows and of fewer
-# tiles than waves, and eight rows per KV head.
+# is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows, of fewer tiles
+# than waves and of the most rows, one and eight rows per KV head; and full suffixes of one round, which stay mixed
+# (N = 16 of 2 rows after 2048 keys) or not (after 8192).
 PREFIX = [dict(N=24, P=8000, S=1000, S_min=0), dict(N=9, P=8191, S=1025, S_min=1), dict(N=13, P=7409, S=34),
-          dict(N=12, P=4100, S=500, S_min=0, Hq=64, dtype="bf16"), dict(N=20, P=5000, S=2048, S_min=1, Hq=16, Hkv=4)]
+          dict(N=12, P=4100, S=500, S_min=0, Hq=64, dtype="bf16"), dict(N=20, P=5000, S=2048, S_min=1),
+          dict(N=9, P=4100, S=300, S_min=0, Hq=32, Hkv=32), dict(N=16, P=2048, S=1024, Hq=32, Hkv=16),
+          dict(N=16, P=8192, S=1024, Hq=32, Hkv=16)]
 PREFIX_PAGED = [dict(N=24, P=8192, S=1000, S_min=0, ps=64, dtype="bf16"),
-                dict(N=11, P=4704, S=700, S_min=0, ps=32, layout="NHD", Hq=64, absent=2)]
+                dict(N=11, P=4704, S=700, S_min=0, ps=32, layout="NHD", Hq=64, absent=2),
+                dict(N=20, P=5024, S=2048, S_min=1, ps=32, dtype="bf16")]
 # DSA decode of batches on indexer workgroups of 1024 positions and each request alone on 256: the last workgroup and
 # tile partly filled, one position past the selection, and the longest request that takes the small ones.
 DSA = [dict(B=30, L=2049), dict(B=9, L=8100, dtype="bf16"), dict(B=5, L=16384), dict(B=17, L=4097)]

@@ -703,7 +703,7 @@ struct PrefixPlan {
 // the same prefix chunks, tile order and merges whatever batch they are in, so a batch row is bit-equal to the same
 // request alone.  N only sets how many row blocks there are (and the row-block width, which groups rows that share
 // a ring without changing any row's arithmetic).
-static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int64_t S) {
+static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int64_t S, bool ragged) {
   PrefixPlan p;
   const int64_t G = Hq / Hkv, R = N * G;
   p.WRp = R <= 128 ? 4 : 8;                                  // waves sharing one ring, 32 rows each
@@ -748,7 +748,19 @@ static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int
   // S = 1024 33.7 / 36.4; N = 6 of 8 rows a head, P = 8192 in NHD pages, S <= 500 25.1 / 31.1; N = 13, P = 7409, S = 34
   // 17.4 / 20.9.  At 128 rows four waves read every prefix tile and the rounds even out: N = 32, P = 4096, S = 256 22.3
   // / 22.0; N = 32, P = 32768, S = 1000 69.5 / 63.0.  Grids of one round stay mixed: N = 8, P = 2048, S = 256 16.4 / 13.7.
-  p.waves = R <= 96 && p.fuse && G <= 8 && p.n_wg_mixed > kDeviceCUs;
+  // Up to 32 rows the gain is as large: 32 KV heads, N = 12, P = 2048, S = 32 16.4 / 24.1.  Over 2600 shapes of 2 to 96
+  // rows waves take 0.82 of the mixed launch's time in the mean, and more than 1.02 in 40 (at most 1.13: N = 32 of 2
+  // rows, 512 suffixes of 2048 after a prefix of 500).
+  // Full suffixes that take one round by themselves and are most of the work leave a second round little to do, and the
+  // merge launch is not won back: 16 KV heads of 2 rows, N = 16, P = 2048, S = 1024 29.7 / 27.4; 8 KV heads of 4, N = 24,
+  // P = 1000, S = 2048 39.1 / 36.3.  They stay mixed where the suffix tiles are at least 5 times the prefix's (10 times,
+  // past 32 rows); below that waves win: N = 16 of 2 rows, P = 8192, S = 1024 37.2 / 38.0; 8 KV heads of 1 row, N = 32,
+  // P = 8192, S = 1024 32.5 / 37.1.  Lengths below S leave the rounds uneven, and waves win again (N = 16 of 2 rows,
+  // P = 2048, S <= 1024 23.0 / 23.6).
+  const int64_t suffix_tiles = n_suffix * (p.chunk_s / kTile), prefix_tiles = Hkv * ((P + kTile - 1) / kTile);
+  const bool one_suffix_round = !ragged && S > 512 && n_suffix <= kDeviceCUs &&
+                                suffix_tiles >= (R <= 32 ? 5 : 10) * prefix_tiles * ((R + 31) / 32);
+  p.waves = R <= 96 && p.fuse && G <= 8 && p.n_wg_mixed > kDeviceCUs && !one_suffix_round;
   return p;
 }
 
@@ -756,7 +768,7 @@ static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int
 template <int kPaged, class V>
 static int prefix_launch(PrefixArgs& a, const void* q, void* out, const void* slens, bool ragged, int64_t N,
                          int64_t Hq, int64_t Hkv, int64_t D, int64_t P, int64_t S, void* workspace, hipStream_t s) {
-  PrefixPlan p = prefix_plan(N, Hq, Hkv, P, S);
+  PrefixPlan p = prefix_plan(N, Hq, Hkv, P, S, ragged);
   a.q = (const f16*)q;
   a.slens = ragged ? (const int*)slens : nullptr;
   a.out = (f16*)out;
@@ -836,9 +848,8 @@ using namespace vmk;
 
 extern "C" size_t vmk_prefix_workspace_size(int64_t N, int64_t Hq, int64_t Hkv, int64_t D, int64_t P, int64_t S,
                                             int64_t ragged) {
-  (void)ragged;
   if (N <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || D != 128 || P < 0 || S < 0 || P + S <= 0) return 0;
-  PrefixPlan p = prefix_plan(N, Hq, Hkv, P, S);
+  PrefixPlan p = prefix_plan(N, Hq, Hkv, P, S, ragged != 0);
   return kWsHead + (p.po_p + p.pml_p + p.po_s + p.pml_s + p.order) * sizeof(float) + 5 * 256;
 }
 
