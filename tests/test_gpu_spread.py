@@ -5,7 +5,8 @@ units of keys out to all waves and folds them in its combine launch, a call that
 Each case runs a batch large enough for the second and every request alone (the first), which must give the same bits,
 and checks the batch against the float64 oracle.  A cache of one split takes one launch without a combine, or units with
 it: the same bits as well.  Sizes: one tile, ends inside the first unit, block and split and just past them, fewer tiles
-than waves, more requests than one scan of the lengths holds, and both row-block forms."""
+than waves, more requests than one scan of the lengths holds, both row-block forms, and 17 to 64 splits to a request (the
+combine over units takes 16 at a time)."""
 import numpy as np
 import pytest
 import torch
@@ -19,12 +20,15 @@ pytestmark = pytest.mark.gpu
 DECODE = [dict(B=70, L=40, L_min=1), dict(B=9, L=2049), dict(B=12, L=4096, L_min=1), dict(B=33, L=1025, L_min=1),
           dict(B=40, L=513, Hq=8, Hkv=1), dict(B=33, L=1280, L_min=1), dict(B=33, L=1281, L_min=1),
           dict(B=33, L=2048, L_min=1, dtype="bf16"), dict(B=9, L=2500, L_min=1, Hq=64, Hkv=8, dtype="bf16"),
-          dict(B=24, L=6000, L_min=1, Hq=48, Hkv=2)]
+          dict(B=24, L=6000, L_min=1, Hq=48, Hkv=2), dict(B=5, L=40000, L_min=32769, Hq=8, Hkv=1),
+          dict(B=3, L=131072, L_min=34000, Hq=8, Hkv=1, dtype="bf16"), dict(B=4, L=34816, L_min=1, Hq=24, Hkv=1)]
 PAGED = [dict(B=20, L=1504, L_min=1, ps=32, dtype="bf16"), dict(B=20, L=2048, L_min=1, ps=64, layout="NHD"),
-         dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16")]
+         dict(B=10, L=2100, L_min=1, ps=64), dict(B=10, L=4100, L_min=1, ps=32, layout="NHD", dtype="bf16"),
+         dict(B=3, L=67584, L_min=33000, Hq=8, Hkv=1, ps=64)]
 SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16), dict(B=9, L=300, k=11, Hq=8, Hkv=2),
         dict(B=9, L=640, k=16), dict(B=9, L=1500, k=16, dtype="bf16"), dict(B=12, L=2048, k=7),
-        dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9)]
+        dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9), dict(B=8, L=70000, k=16, Hq=4, Hkv=1),
+        dict(B=4, L=40000, k=3, Hq=8, Hkv=1, dtype="bf16")]
 # Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone, which
 # is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows, of fewer tiles
 # than waves and of the most rows, one and eight rows per KV head; and full suffixes of one round, which stay mixed
