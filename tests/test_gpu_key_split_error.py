@@ -1,0 +1,41 @@
+"""Error of attention over few splits against float64, in fp16, for groups of 17 to 64 rows and of up to 128 keys per row.
+
+P and the result are each rounded to fp16 once.  A rounding's relative error is uniform within half a unit of the last
+place, over mantissas spread as 1/m: 2^-10 / sqrt(12) / sqrt(3 / (2 ln 2)) = 1.92e-4 in the 2-norm, so two give 2.71e-4 and
+a third, of the splits' rows, 3.32e-4 (the measured figures lie 5 % above).  The bound is that of two and a half roundings."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from vmk.ops import decode, spec
+
+pytestmark = pytest.mark.gpu
+
+BOUND = 1.05 * 2.5 ** 0.5 * 1.92e-4
+
+
+def rel(out, ref):
+    return float(np.linalg.norm(out.double().cpu().numpy() - ref) / np.linalg.norm(ref))
+
+
+# One to a few requests (units) and batches that fill the chip (splits), on both sides of a tile's and a split's end.
+@pytest.mark.parametrize("shape", [dict(B=1, L=5000, k=12), dict(B=1, L=2500, k=5), dict(B=2, L=4096, k=8),
+                                   dict(B=1, L=8192, k=16), dict(B=9, L=4097, k=16), dict(B=12, L=2049, k=6),
+                                   dict(B=20, L=3333, k=7)])
+def test_verify_error(shape):
+    import spec_mi355x
+    inp = spec.make_inputs(shape, seed=71, dist="chain", device="cuda")
+    e = rel(spec_mi355x.kernel(**inp), oracle.spec.ref64(**inp))
+    print(f"{shape} {e:.3e}", flush=True)
+    assert e <= BOUND
+
+
+@pytest.mark.parametrize("shape", [dict(B=40, L=8192, L_min=2049, Hq=64, Hkv=1), dict(B=2, L=4000, L_min=3000, Hq=64, Hkv=2),
+                                   dict(B=30, L=3072, L_min=2049, Hq=48, Hkv=2)])
+def test_ragged_decode_error(shape):
+    import vmk
+    inp = decode.make_inputs(shape, seed=72, device="cuda")
+    e = rel(vmk.decode(**inp), oracle.decode.ref64(**inp))
+    print(f"{shape} {e:.3e}", flush=True)
+    assert e <= BOUND

@@ -712,10 +712,10 @@ static_assert(kAttnSlotsEnd <= kAttnSmemBytes, "merge slots must fit in the stag
 struct NoRow {
   __device__ __forceinline__ float* operator()(int) const { return nullptr; }
 };
-template <int WR, int WK, int NSW = 2, class V = half8, bool kFold = false, class Src, class QRow, class PT,
+template <int WR, int WK, int NSW = 2, class V = half8, bool kFold = false, class Src, class QRow, class PO,
           class ORow = NoRow>
 __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow, int nrows, int kbeg, int ntiles,
-                                          PT* po, float* pml, int unit = 0, ORow orow = ORow()) {
+                                          PO po, float* pml, int unit = 0, ORow orow = ORow()) {
   constexpr bool kFinal = !std::is_same_v<ORow, NoRow>;
   static_assert(WR * WK == 4 && WK > 1 && WR * WK * NSW <= 8, "four waves, rings within the stage memory");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -750,7 +750,7 @@ __device__ __forceinline__ void attend_wg(char* smem, const Src& src, QRow qrow,
     st.l += xor32(st.l);
   }
   const int nvalid = nrows - wr * 32;
-  PT* pob = po + (size_t)wr * 32 * 128;
+  const PO pob = po + (size_t)wr * 32 * 128;
   float* pmlb = pml + wr * 32 * 2;
   {
     __syncthreads();                                        // every walk is done: the rings become slots

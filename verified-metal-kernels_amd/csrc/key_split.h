@@ -25,13 +25,14 @@ struct KeySplitArgs {
   const uint32_t* bits;    // (B, kd, W), or null: every cache position visible to every query row (plain decode)
   const int* lens;         // (B,) cache positions in use per batch entry (clamped to [kd, L]), or null: all L
   const int* pages;        // paged: (B, max_pages) page table
-  // Partials, [grp - g0][row block][slots][rows_s][128] and their (m, l) pairs: splits as normalised O rows of part_t
-  // (one row block), or units as fp32 sums (row blocks of 32 rows).
+  // Partials, [grp - g0][row block][slots][rows_s][128] and their (m, l) pairs: splits as normalised O rows of part_t, or
+  // of fp32 where split_wide() (one row block), or units as fp32 sums (row blocks of 32 rows).
   void* part_o;
   float* part_ml;
   void* out;               // (B, kd, Hq, 128)
   int B, kd, Hq, Hkv, G, L, W;
   int ps, max_pages, num_pages;
+  int esize;               // bytes that an element of a split's rows is given (fp16 rows fill half of 4)
   int nrb, slots, rows_s;  // row blocks of a group; splits or units per (group, row block), at most; rows of one partial
   int g0, ngrp;            // groups of this launch (with lens: all of them)
   int logw;                // units: log2 of the shares the line of tiles is cut into (four waves each)
@@ -59,6 +60,17 @@ template <class N>
 __host__ __device__ inline N group_splits(int rows, N n) {
   const int s = split_log2(rows, n);
   return (n + (1 << s) - 1) >> s;
+}
+
+// Whether a group's splits stay fp32 for fp16 inputs: groups of more than 16 rows and of up to 128 keys per row, which
+// 2048 keys cut into two to four.  As one split their rows would be rounded once, so rounding the splits would add an
+// error that one split does not have (12 drafts over 5000 keys, relative error 2.92e-4 as one split, 3.53e-4 as three in
+// fp16, 2.88e-4 in fp32).  Longer groups have several splits of either size and round them to fp16 as ever.
+// The rows are twice the bytes: 16 drafts, 8 requests of 8192 keys 51.1 us for 51.0, 9 drafts of 5000 35.8 for 35.5, 16
+// drafts, 32 requests of 8192 keys 224 for 214.
+template <class N>
+__host__ __device__ inline bool split_wide(int rows, N n) {
+  return rows > 16 && n > 2048 && n <= 128 * rows;
 }
 
 // log2 of the tiles of a unit of a group with nt key tiles: about 64 units to a group, at least four or eight tiles (a
@@ -460,7 +472,13 @@ __global__ __launch_bounds__(256) void key_split_kernel(KeySplitArgs a) {
     return a.q + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
   };
   typedef part_t<elem_t<V>> PT;
-  PT* po = reinterpret_cast<PT*>(a.part_o) + (size_t)item * a.rows_s * 128;
+  constexpr bool kDual = kSrc == kStreamContig && sizeof(PT) == 2;   // pages have at most 16 rows
+  char* const po_b = reinterpret_cast<char*>(a.part_o) + (size_t)item * a.rows_s * 128 * a.esize;
+  std::conditional_t<kDual, HalfOrFloat, PT*> po;
+  if constexpr (kDual)
+    po = HalfOrFloat{po_b, split_wide(R, n)};
+  else
+    po = reinterpret_cast<PT*>(po_b);
   float* pml = a.part_ml + (size_t)item * a.rows_s * 2;
   auto orow = [&](int r) {
     const int i = r / a.G, gg = r - i * a.G;
@@ -509,23 +527,29 @@ __global__ __launch_bounds__(128) void key_split_combine_kernel(KeySplitArgs a) 
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int n = group_splits(R, stream_len_uniform(a, b));
+  const int len = stream_len_uniform(a, b), n = group_splits(R, len);
   const int i = row / a.G, gg = row - i * a.G;
-  typedef part_t<E> PT;
   E* out = reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128;
-  if (n == 1) {
-    const size_t base = (size_t)grel * a.slots * a.rows_s + row;
-    const float x = (float)reinterpret_cast<const PT*>(a.part_o)[base * 128 + threadIdx.x];
-    out[threadIdx.x] = (E)(a.part_ml[base * 2 + 1] == 0.f ? __builtin_nanf("") : x);
-    return;
-  }
-  combine_row<128, 1, PT>(n,
-                          [&](int s, const float*& ml, const PT*& o) {
-                            const size_t base = ((size_t)grel * a.slots + s) * a.rows_s + row;
-                            ml = a.part_ml + base * 2;
-                            o = reinterpret_cast<const PT*>(a.part_o) + base * 128;
-                          },
-                          out);
+  auto merge = [&](auto t) {
+    typedef decltype(t) T;
+    auto part = [&](int s, const float*& ml, const T*& o) {
+      const size_t item = (size_t)grel * a.slots + s;
+      ml = a.part_ml + (item * a.rows_s + row) * 2;
+      o = reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.part_o) + item * a.rows_s * 128 * a.esize) + row * 128;
+    };
+    if (n == 1) {
+      const float* ml;
+      const T* o;
+      part(0, ml, o);
+      out[threadIdx.x] = (E)(ml[1] == 0.f ? __builtin_nanf("") : (float)o[threadIdx.x]);
+    } else {
+      combine_row<128, 1, T>(n, part, out);
+    }
+  };
+  if (sizeof(part_t<E>) == 2 && split_wide(R, len))
+    merge(float());
+  else
+    merge(part_t<E>());
 }
 
 // The same for many rows (at least kSplitVecRows): one wave per 4 rows, 16 lanes per row, each lane 8 head-dims loaded
@@ -539,28 +563,36 @@ __global__ __launch_bounds__(64) void key_split_combine_vec_kernel(KeySplitArgs 
   if (rowg >= a.ngrp * R) return;                           // a whole row group of lanes
   const int grel = rowg / R, row = rowg - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int n = group_splits(R, stream_len(a, b));
+  const int len = stream_len(a, b), n = group_splits(R, len);
   const int i = row / a.G, gg = row - i * a.G;
-  typedef part_t<E> PT;
   E* out = reinterpret_cast<E*>(a.out) + ((size_t)(b * a.kd + i) * a.Hq + h * a.G + gg) * 128 + 8 * c;
-  if (n == 1) {
-    const size_t base = (size_t)grel * a.slots * a.rows_s + row;
-    Part8<PT> o;
-    o.load(reinterpret_cast<const PT*>(a.part_o) + base * 128 + 8 * c);
-    const bool none = a.part_ml[base * 2 + 1] == 0.f;
-    float x[8];
+  auto merge = [&](auto t) {
+    typedef decltype(t) T;
+    auto part = [&](int s, const float*& ml, const T*& o) {
+      const size_t item = (size_t)grel * a.slots + s;
+      ml = a.part_ml + (item * a.rows_s + row) * 2;
+      o = reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.part_o) + item * a.rows_s * 128 * a.esize) +
+          row * 128 + 8 * c;
+    };
+    if (n == 1) {
+      const float* ml;
+      const T* op;
+      part(0, ml, op);
+      Part8<T> o;
+      o.load(op);
+      const bool none = ml[1] == 0.f;
+      float x[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) x[k] = none ? __builtin_nanf("") : o.get(k);
-    store_out8(out, x, 1.f);
-    return;
-  }
-  combine_vec<PT>(n,
-                  [&](int s, const float*& ml, const PT*& o) {
-                    const size_t base = ((size_t)grel * a.slots + s) * a.rows_s + row;
-                    ml = a.part_ml + base * 2;
-                    o = reinterpret_cast<const PT*>(a.part_o) + base * 128 + 8 * c;
-                  },
-                  out);
+      for (int k = 0; k < 8; ++k) x[k] = none ? __builtin_nanf("") : o.get(k);
+      store_out8(out, x, 1.f);
+    } else {
+      combine_vec<T>(n, part, out);
+    }
+  };
+  if (sizeof(part_t<E>) == 2 && split_wide(R, len))
+    merge(float());
+  else
+    merge(part_t<E>());
 }
 
 // One output row per workgroup from stored units: lane group s (16 lanes, eight head-dims each) folds the units of
@@ -570,14 +602,16 @@ template <class E>
 __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) {
   typedef part_t<E> PT;
   __shared__ float redm[4], sm[16], sl[16];
-  __shared__ __attribute__((aligned(16))) PT so[16][128];
+  __shared__ __attribute__((aligned(16))) float so[16][128];   // rounded to PT, but for wide splits
   const int tid = threadIdx.x, c = tid & 15, s = tid >> 4;
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
   const int g = a.g0 + grel, b = g / a.Hkv, h = g - b * a.Hkv;
-  const int len = stream_len_uniform(a, b), nt = tiles_of(len), n = group_units(R, nt), q = split_waves(R);   // q: waves of a split
-  const int per = 1 << (split_log2(R, len) - 5 - split_waves_log2(R) - unit_log2(R, nt));   // units of a wave in a split
+  const int len = stream_len_uniform(a, b), nt = tiles_of(len), n = group_units(R, nt);
+  // Waves of a split, and units of a wave in it.
+  const int q = split_waves(R), per = 1 << (split_log2(R, len) - 5 - split_waves_log2(R) - unit_log2(R, nt));
   const int nsplit = group_splits(R, len);
+  const bool wide = sizeof(PT) == 4 || split_wide(R, len);
   const size_t p0 = (((size_t)grel * a.nrb + (row >> 5)) * a.slots) * a.rows_s + (row & 31);
   const float* po = reinterpret_cast<const float*>(a.part_o) + 8 * c;
   auto ml_of = [&](int i) { return *reinterpret_cast<const float2*>(a.part_ml + (p0 + (size_t)i * a.rows_s) * 2); };
@@ -647,8 +681,14 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
       sl[s] = l;
     }
 #pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      acc[k] *= inv;
+      asm("" : "+v"(acc[k]));                               // rounded to fp32 first, not fused with the conversion
+      if (!wide) acc[k] = (float)(PT)acc[k];
+    }
+#pragma unroll
     for (int k = 0; k < 8; k += 4)
-      store_part4(&so[s][8 * c + k], floatx4{acc[k] * inv, acc[k + 1] * inv, acc[k + 2] * inv, acc[k + 3] * inv});
+      store_part4(&so[s][8 * c + k], floatx4{acc[k], acc[k + 1], acc[k + 2], acc[k + 3]});
   };
   float M = kNegInf;
   if (nsplit > 16) {                                        // the largest m before the first weight
@@ -674,13 +714,13 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
       for (int j = 0; j < ns; ++j) {
         const float w = part_weight(float2{sm[j], sl[j]}, M);
         den += w;
-        num += w * (float)so[j][tid];
+        num += w * so[j][tid];
       }
     }
   }
   if (tid >= 128) return;
   if (nsplit == 1) {                                        // the split is the result, as key_split_kernel writes it
-    num = sl[0] == 0.f ? __builtin_nanf("") : (float)so[0][tid];
+    num = sl[0] == 0.f ? __builtin_nanf("") : so[0][tid];
     den = 1.f;
   }
   const int di = row / a.G, gg = row - di * a.G;
@@ -692,15 +732,16 @@ struct KeySplitPlan {
   int rows, nsplit;        // nsplit: splits of a group of L keys
   bool units;
   int nrb, slots, rows_s;
+  size_t esize;            // bytes for an element of a partial row
   size_t grp_rows;         // partial rows of one group
 };
 
-// Bytes of the O rows (to the next 256-byte boundary) and of all partials of ngrp groups; e: bytes of a split's element.
-inline size_t key_split_ml_offset(const KeySplitPlan& p, int64_t ngrp, size_t e) {
-  return (ngrp * p.grp_rows * 128 * (p.units ? sizeof(float) : e) + 255) / 256 * 256;
+// Bytes of the O rows (to the next 256-byte boundary) and of all partials of ngrp groups.
+inline size_t key_split_ml_offset(const KeySplitPlan& p, int64_t ngrp) {
+  return (ngrp * p.grp_rows * 128 * p.esize + 255) / 256 * 256;
 }
-inline size_t key_split_bytes(const KeySplitPlan& p, int64_t ngrp, size_t e) {
-  return key_split_ml_offset(p, ngrp, e) + ngrp * p.grp_rows * 2 * sizeof(float);
+inline size_t key_split_bytes(const KeySplitPlan& p, int64_t ngrp) {
+  return key_split_ml_offset(p, ngrp) + ngrp * p.grp_rows * 2 * sizeof(float);
 }
 
 // The most splits and rows of a unit launch.
@@ -719,8 +760,8 @@ inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
 // 15.3, of 2048 15.0 and 18.6.
 //
 // ragged: a group may be shorter than L (and have more splits than one of L keys, where the split size steps up).
-// room: bytes there are for the partials of all groups (a split's element takes e); units that need more stay splits,
-// with the same bits.
+// e: bytes of an element of a split's row (fp32 for fp16 inputs where split_wide() can hold).  room: bytes there are for
+// the partials of all groups; units that need more stay splits, with the same bits.
 inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged, size_t e, size_t room) {
   KeySplitPlan p;
   p.rows = (int)rows;
@@ -733,10 +774,11 @@ inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool r
     p.nrb = p.units ? (int)((rows + 31) / 32) : 1;
     p.rows_s = rows <= 32 || !p.units ? (int)rows : 32;
     p.slots = (int)(p.units ? unit_slots((int)rows, L) : ragged ? split_slots((int)rows, L) : p.nsplit);
+    p.esize = p.units || (rows > 16 && (ragged ? L > 2048 : split_wide((int)rows, L))) ? sizeof(float) : e;
     p.grp_rows = (size_t)p.nrb * p.slots * p.rows_s;
   };
   lay_out();
-  if (p.units && key_split_bytes(p, ngrp, e) > room) {
+  if (p.units && key_split_bytes(p, ngrp) > room) {
     p.units = false;
     lay_out();
   }
@@ -763,8 +805,8 @@ template <int kSrc, bool kBits, class V>
 inline int key_split_launch(KeySplitArgs a, const KeySplitPlan& p, void* partials, hipStream_t s) {
   typedef elem_t<V> E;
   a.part_o = partials;
-  a.part_ml = reinterpret_cast<float*>((char*)partials + key_split_ml_offset(p, a.ngrp, sizeof(part_t<E>)));
-  a.nrb = p.nrb; a.slots = p.slots; a.rows_s = p.rows_s;
+  a.part_ml = reinterpret_cast<float*>((char*)partials + key_split_ml_offset(p, a.ngrp));
+  a.nrb = p.nrb; a.slots = p.slots; a.rows_s = p.rows_s; a.esize = (int)p.esize;
   const int64_t rows = (int64_t)a.ngrp * p.rows;
   if (!p.units) {
     prof_before(kKSpecPartial, s);

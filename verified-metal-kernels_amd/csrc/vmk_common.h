@@ -56,6 +56,18 @@ __device__ __forceinline__ void store_part4(bf16* p, floatx4 v) {
   typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
   *reinterpret_cast<bf16x4*>(p) = bf16x4{(bf16)v[0], (bf16)v[1], (bf16)v[2], (bf16)v[3]};
 }
+// Rows of fp16 or, where wide, of fp32: a pointer to the first, moved by elements.
+struct HalfOrFloat {
+  char* p;
+  bool wide;
+  __device__ __forceinline__ HalfOrFloat operator+(size_t n) const { return HalfOrFloat{p + (n << (wide ? 2 : 1)), wide}; }
+};
+__device__ __forceinline__ void store_part4(HalfOrFloat p, floatx4 v) {
+  if (p.wide)
+    store_part4(reinterpret_cast<float*>(p.p), v);
+  else
+    store_part4(reinterpret_cast<f16*>(p.p), v);
+}
 // The same as non-temporal stores, for partials that are read back only by a later launch: they stream to memory
 // instead of waiting in L2 for the end-of-kernel writeback (C2's prefix partials -2 %; partials that a combine reads
 // right after, as C3's, lose by it).

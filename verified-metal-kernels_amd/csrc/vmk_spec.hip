@@ -243,7 +243,7 @@ static int spec_call(const void* q, const void* k, const void* v, const void* ma
   constexpr size_t e = sizeof(part_t<elem_t<V>>);
   const KeySplitPlan p = key_split_plan(groups, R, L, lens != nullptr, e, room);
   int64_t steps = 1, step = groups;
-  while (key_split_bytes(p, step, e) > room) {
+  while (key_split_bytes(p, step) > room) {
     VMK_CHECK(step > 1, "no room for the partials of one KV head");
     step = (groups + steps) / (steps + 1);
     ++steps;
