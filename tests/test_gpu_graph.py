@@ -89,3 +89,29 @@ def test_graph_replays_equal_eager_dsa_project():
                 assert torch.equal(got, want), rep
         run(inps[rep % 2])                              # eager work between replays
         torch.cuda.synchronize()
+
+
+def test_capture_after_one_eager_call_of_the_largest_batch(monkeypatch):
+    """One eager call of the largest batch and cache leaves a workspace that every smaller call fits, so a smaller one
+    can be captured afterwards (a call of few requests stores units, a large one splits only)."""
+    import vmk
+    from vmk import api
+    from vmk.ops import decode as dec
+    monkeypatch.setattr(api, "_ws", {})
+    monkeypatch.setattr(api, "_captured", set())
+    big = dec.make_inputs(dict(B=64, L=2048), seed=81, device="cuda")
+    small = dec.make_inputs(dict(B=8, L=2048), seed=82, device="cuda")
+    print("capture after the largest batch", flush=True)
+    vmk.decode(**big)
+    torch.cuda.synchronize()
+    out = torch.empty_like(small["q"])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        vmk.decode(**small, out=out)
+    want = vmk.decode(**small)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16))
+        vmk.decode(**big)
