@@ -1,8 +1,8 @@
-"""Error of attention over few splits against float64, in fp16, for groups of 17 to 64 rows and of up to 128 keys per row.
+"""Error of attention over few splits against float64, in fp16, for groups of 17 to 64 rows and up to 128 keys per row.
 
 P and the result are each rounded to fp16 once.  A rounding's relative error is uniform within half a unit of the last
-place, over mantissas spread as 1/m: 2^-10 / sqrt(12) / sqrt(3 / (2 ln 2)) = 1.92e-4 in the 2-norm, so two give 2.71e-4 and
-a third, of the splits' rows, 3.32e-4 (the measured figures lie 5 % above).  The bound is that of two and a half roundings."""
+place, over mantissas spread as 1/m: 2^-10 / sqrt(12) / sqrt(3 / (2 ln 2)) = 1.92e-4 in the 2-norm, so two give 2.71e-4
+and a third, of the splits' rows, 3.32e-4 (the measured figures lie 5 % above).  The bound is that of two and a half."""
 import numpy as np
 import pytest
 import torch
@@ -31,7 +31,8 @@ def test_verify_error(shape):
     assert e <= BOUND
 
 
-@pytest.mark.parametrize("shape", [dict(B=40, L=8192, L_min=2049, Hq=64, Hkv=1), dict(B=2, L=4000, L_min=3000, Hq=64, Hkv=2),
+@pytest.mark.parametrize("shape", [dict(B=40, L=8192, L_min=2049, Hq=64, Hkv=1),
+                                   dict(B=2, L=4000, L_min=3000, Hq=64, Hkv=2),
                                    dict(B=30, L=3072, L_min=2049, Hq=48, Hkv=2)])
 def test_ragged_decode_error(shape):
     import vmk

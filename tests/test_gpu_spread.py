@@ -5,8 +5,8 @@ units of keys out to all waves and folds them in its combine launch, a call that
 Each case runs a batch large enough for the second and every request alone (the first), which must give the same bits,
 and checks the batch against the float64 oracle.  A cache of one split takes one launch without a combine, or units with
 it: the same bits as well.  Sizes: one tile, ends inside the first unit, block and split and just past them, fewer tiles
-than waves, more requests than one scan of the lengths holds, both row-block forms, and 17 to 64 splits to a request (the
-combine over units takes 16 at a time)."""
+than waves, more requests than one scan of the lengths holds, both row-block forms, and 17 to 64 splits to a request
+(the combine over units takes 16 at a time)."""
 import numpy as np
 import pytest
 import torch
@@ -29,10 +29,10 @@ SPEC = [dict(B=9, L=2049, k=8), dict(B=5, L=8300, k=5), dict(B=10, L=4200, k=16)
         dict(B=9, L=640, k=16), dict(B=9, L=1500, k=16, dtype="bf16"), dict(B=12, L=2048, k=7),
         dict(B=6, L=16500, k=2), dict(B=5, L=20000, k=9), dict(B=8, L=70000, k=16, Hq=4, Hkv=1),
         dict(B=4, L=40000, k=3, Hq=8, Hkv=1, dtype="bf16")]
-# Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone, which
-# is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows, of fewer tiles
-# than waves and of the most rows, one and eight rows per KV head; and full suffixes of one round, which stay mixed
-# (N = 16 of 2 rows after 2048 keys) or not (after 8192).
+# Shared prefix as single waves (two rounds of the mixed launch, up to 96 rows per KV head) and each request alone,
+# which is not: one, two and three row blocks, the last row, tile and chunk partly filled, suffixes of no rows, of fewer
+# tiles than waves and of the most rows, one and eight rows per KV head; and full suffixes of one round, which stay
+# mixed (N = 16 of 2 rows after 2048 keys) or not (after 8192).
 PREFIX = [dict(N=24, P=8000, S=1000, S_min=0), dict(N=9, P=8191, S=1025, S_min=1), dict(N=13, P=7409, S=34),
           dict(N=12, P=4100, S=500, S_min=0, Hq=64, dtype="bf16"), dict(N=20, P=5000, S=2048, S_min=1),
           dict(N=9, P=4100, S=300, S_min=0, Hq=32, Hkv=32), dict(N=16, P=2048, S=1024, Hq=32, Hkv=16),

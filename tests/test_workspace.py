@@ -85,9 +85,9 @@ def test_error_codes_are_kept():
     assert lib.VmkError("y").code is None
 
 
-@pytest.mark.parametrize("op,heads", [("decode", (32, 8)), ("decode", (16, 1)), ("decode", (96, 4)), ("decode", (64, 1)),
-                                      ("paged", (32, 8)), ("paged", (8, 1)),
-                                      (2, (32, 8)), (7, (32, 8)), (8, (32, 8)), (9, (32, 8)), (16, (32, 8)), (16, (4, 1)),
+@pytest.mark.parametrize("op,heads", [("decode", (32, 8)), ("decode", (16, 1)), ("decode", (96, 4)),
+                                      ("decode", (64, 1)), ("paged", (32, 8)), ("paged", (8, 1)), (2, (32, 8)),
+                                      (7, (32, 8)), (8, (32, 8)), (9, (32, 8)), (16, (32, 8)), (16, (4, 1)),
                                       (64, (32, 8))])
 def test_sizes_grow_with_the_batch_and_the_cache(op, heads):
     """A workspace sized for the largest batch and cache serves every smaller call: the sizes never fall as either

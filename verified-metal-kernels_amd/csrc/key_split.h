@@ -25,8 +25,8 @@ struct KeySplitArgs {
   const uint32_t* bits;    // (B, kd, W), or null: every cache position visible to every query row (plain decode)
   const int* lens;         // (B,) cache positions in use per batch entry (clamped to [kd, L]), or null: all L
   const int* pages;        // paged: (B, max_pages) page table
-  // Partials, [grp - g0][row block][slots][rows_s][128] and their (m, l) pairs: splits as normalised O rows of part_t, or
-  // of fp32 where split_wide() (one row block), or units as fp32 sums (row blocks of 32 rows).
+  // Partials, [grp - g0][row block][slots][rows_s][128] and their (m, l) pairs: splits as normalised O rows of part_t,
+  // or of fp32 where split_wide() (one row block), or units as fp32 sums (row blocks of 32 rows).
   void* part_o;
   float* part_ml;
   void* out;               // (B, kd, Hq, 128)
@@ -64,10 +64,10 @@ __host__ __device__ inline N group_splits(int rows, N n) {
 
 // Whether a group's splits stay fp32 for fp16 inputs: groups of more than 16 rows and of up to 128 keys per row, which
 // 2048 keys cut into two to four.  As one split their rows would be rounded once, so rounding the splits would add an
-// error that one split does not have (12 drafts over 5000 keys, relative error 2.92e-4 as one split, 3.53e-4 as three in
-// fp16, 2.88e-4 in fp32).  Longer groups have several splits of either size and round them to fp16 as ever.
-// The rows are twice the bytes: 16 drafts, 8 requests of 8192 keys 51.1 us for 51.0, 9 drafts of 5000 35.8 for 35.5, 16
-// drafts, 32 requests of 8192 keys 224 for 214.
+// error that one split does not have (12 drafts over 5000 keys, relative error 2.92e-4 as one split, 3.53e-4 as three
+// in fp16, 2.88e-4 in fp32).  Longer groups have several splits of either size and round them to fp16 as ever. The rows
+// are twice the bytes: 16 drafts, 8 requests of 8192 keys 51.1 us for 51.0, 9 drafts of 5000 35.8 for 35.5, 16 drafts,
+// 32 requests of 8192 keys 224 for 214.
 template <class N>
 __host__ __device__ inline bool split_wide(int rows, N n) {
   return rows > 16 && n > 2048 && n <= 128 * rows;
@@ -444,8 +444,9 @@ struct SplitSrc {
 };
 
 // kFinal: no group has more than one split; its rows are the result and no combine launch follows.  (The combines of
-// larger caches write a group's only split as it is, too: the same bits.)  Decode of one and 16 requests of 1000 keys 15.3 and
-// 16.6 us with the combine, 12.2 and 13.7 without; verification of 16 drafts in four of 2000 keys 35.3 and 32.4.
+// larger caches write a group's only split as it is, too: the same bits.)  Decode of one and 16 requests of 1000 keys
+// 15.3 and 16.6 us with the combine, 12.2 and 13.7 without; verification of 16 drafts in four of 2000 keys 35.3 and
+// 32.4.
 //
 // Ragged lengths: workgroup id i runs on XCD i modulo 8, so with eight splits to a group (16384 positions) split 7 of
 // every group, which only the longest requests have, would run on one XCD and split 0, which all have, on another.  The
@@ -535,7 +536,8 @@ __global__ __launch_bounds__(128) void key_split_combine_kernel(KeySplitArgs a) 
     auto part = [&](int s, const float*& ml, const T*& o) {
       const size_t item = (size_t)grel * a.slots + s;
       ml = a.part_ml + (item * a.rows_s + row) * 2;
-      o = reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.part_o) + item * a.rows_s * 128 * a.esize) + row * 128;
+      o = reinterpret_cast<const T*>(reinterpret_cast<const char*>(a.part_o) + item * a.rows_s * 128 * a.esize) +
+          row * 128;
     };
     if (n == 1) {
       const float* ml;
@@ -759,8 +761,8 @@ inline int64_t unit_max_rows(int rows) { return rows > 32 ? 1024 : 512; }
 // and eight requests of 1000 keys 15.3 and 14.7 us as units, 12.2 and 12.1 as a split; of one of 1500 keys 15.0 and
 // 15.3, of 2048 15.0 and 18.6.
 //
-// ragged: a group may be shorter than L (and have more splits than one of L keys, where the split size steps up).
-// e: bytes of an element of a split's row (fp32 for fp16 inputs where split_wide() can hold).  room: bytes there are for
+// ragged: a group may be shorter than L (and have more splits than one of L keys, where the split size steps up). e:
+// bytes of an element of a split's row (fp32 for fp16 inputs where split_wide() can hold).  room: bytes there are for
 // the partials of all groups; units that need more stay splits, with the same bits.
 inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool ragged, size_t e, size_t room) {
   KeySplitPlan p;
@@ -785,10 +787,10 @@ inline KeySplitPlan key_split_plan(int64_t ngrp, int64_t rows, int64_t L, bool r
   return p;
 }
 
-// Bytes of partials, in fp32, that hold those of any call of up to ngrp groups over caches of up to L positions, so that
-// one workspace sized for the largest call serves the smaller ones: a call of fewer groups may take units, which need
-// more than the splits of many groups do.  A unit launch has at most unit_max_splits() splits and unit_max_rows() rows,
-// and a group at most 64 units or split_waves() to a split.
+// Bytes of partials, in fp32, that hold those of any call of up to ngrp groups over caches of up to L positions, so
+// that one workspace sized for the largest call serves the smaller ones: a call of fewer groups may take units, which
+// need more than the splits of many groups do.  A unit launch has at most unit_max_splits() splits and unit_max_rows()
+// rows, and a group at most 64 units or split_waves() to a split.
 inline size_t key_split_max_bytes(int64_t ngrp, int64_t rows64, int64_t L) {
   const int rows = (int)rows64, q = split_waves(rows);
   const int64_t cap = std::min(ngrp, std::min(unit_max_splits(rows), unit_max_rows(rows) / rows));

@@ -60,7 +60,9 @@ __device__ __forceinline__ void store_part4(bf16* p, floatx4 v) {
 struct HalfOrFloat {
   char* p;
   bool wide;
-  __device__ __forceinline__ HalfOrFloat operator+(size_t n) const { return HalfOrFloat{p + (n << (wide ? 2 : 1)), wide}; }
+  __device__ __forceinline__ HalfOrFloat operator+(size_t n) const {
+    return HalfOrFloat{p + (n << (wide ? 2 : 1)), wide};
+  }
 };
 __device__ __forceinline__ void store_part4(HalfOrFloat p, floatx4 v) {
   if (p.wide)

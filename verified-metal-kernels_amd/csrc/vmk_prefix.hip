@@ -14,9 +14,10 @@
 //   the log-sum-exp merge of its prefix and suffix partials.
 // With at most 128 rows per KV head, launches 1 and 2 are one grid (prefix_mixed_kernel; with at most 32 rows and
 // more items than CUs, its prefix items are single-wave units packed 2 or 4 per workgroup); when that grid has more
-// workgroups than CUs, single-wave workgroups and a merge launch (prefix_waves_kernel).  Its whole-suffix items
-// wait for their KV head's prefix partials and merge them in the same launch when G <= 4 and there are at most 32
-// prefix chunks (mfuse below); otherwise prefix_merge_kernel does the whole-suffix merges.
+// workgroups than CUs, up to 96 rows, mostly single-wave workgroups and a merge launch (prefix_waves_kernel, by the rule
+// in prefix_plan).  The mixed launch's whole-suffix items wait for their KV head's prefix partials and merge them in
+// the same launch when G <= 4 and there are at most 32 prefix chunks (mfuse below); otherwise prefix_merge_kernel does
+// the whole-suffix merges.
 #include "attn_core.h"
 #include "vmk_internal.h"
 
@@ -143,9 +144,9 @@ template <class PT> __device__ __forceinline__ const PT* prefix_po(const PrefixA
 }
 
 // Final output of request n's G rows of KV head h: log-sum-exp merge of the suffix partial (lpo: normalised rows of
-// 128, lpml (m, l) pairs) with the prefix partials of those rows, each weighted exp2(m - M) * l.  One wave per row, two head-dims per lane.
-// Lane s holds the (m, l) of prefix partial b0 + s; the O rows are fetched 16 partials at a time with independent
-// loads (one memory round trip per 16), weighted with the lane-broadcast weights.
+// 128, lpml (m, l) pairs) with the prefix partials of those rows, each weighted exp2(m - M) * l.  One wave per row, two
+// head-dims per lane. Lane s holds the (m, l) of prefix partial b0 + s; the O rows are fetched 16 partials at a time
+// with independent loads (one memory round trip per 16), weighted with the lane-broadcast weights.
 template <class E>
 __device__ void merge_prefix_rows(const PrefixArgs& a, const part_t<E>* lpo, const float* lpml, int n, int h) {
   typedef part_t<E> PT;
@@ -510,17 +511,17 @@ __global__ __launch_bounds__(256) void prefix_mixed_kernel(PrefixArgs a) {
   }
 }
 
-// Up to 128 rows per KV head and more items than the mixed launch runs in one round: the same work one wave at a time.
-// A workgroup is one wave with a two-stage ring (32 KB of LDS, so up to five share a CU and the dispatcher hands out the
-// next as each ends), and does a prefix unit (KV head, 32 of its N * G rows, prefix chunk) or a suffix piece (request,
-// KV head, one of the four interleaved tile sequences that a suffix item's waves walk).  With 128 KB workgroups a CU
-// holds one at a time, and a latency-bound prefix item and a suffix item ran one after the other.  Pieces are stored as
-// the walk leaves them (fp32 sums); prefix_waves_merge_kernel merges the four of a suffix as attend_wg does, and then
-// the prefix partials as every other path does, so the bits are theirs.  A chunk's row blocks run on one XCD (workgroup
-// id modulo 8), whose L2 then serves all but the first read of a tile.  Bound by latency (a tile takes a wave about
-// 1.1 us, a wave's start 4 us): N = 24, P = 8192 in pages, S <= 1000: 25.7 us and 5.4 for the merge, against 34.5 for the
-// mixed launch.  Three or four stages (three or two waves per CU) 32.9 and 43.5 us a call, five waves per CU (256
-// registers, spilled) 37.0, against 30.5.
+// Up to 96 rows per KV head and more items than the mixed launch runs in one round: the same work one wave at a time. A
+// workgroup is one wave with a two-stage ring (32 KB of LDS; four share a CU, one per SIMD by registers, and the
+// dispatcher hands out the next as each ends), and does a prefix unit (KV head, 32 of its N * G rows, prefix chunk) or
+// a suffix piece (request, KV head, one of the four interleaved tile sequences that a suffix item's waves walk).  With
+// 128 KB workgroups a CU holds one at a time, and a latency-bound prefix item and a suffix item ran one after the
+// other. Pieces are stored as the walk leaves them (fp32 sums); prefix_waves_merge_kernel merges the four of a suffix
+// as attend_wg does, and then the prefix partials as every other path does, so the bits are theirs.  A chunk's row
+// blocks run on one XCD (workgroup id modulo 8), whose L2 then serves all but the first read of a tile.  Bound by
+// latency (a tile takes a wave about 1.1 us, a wave's start 4 us): N = 24, P = 8192 in pages, S <= 1000: 25.7 us and
+// 5.4 for the merge, against 34.5 for the mixed launch.  Three or four stages (three or two waves per CU) 32.9 and 43.5
+// us a call, five waves per CU (256 registers, spilled) 37.0, against 30.5.
 constexpr int kWaveStages = 2;
 template <int kPaged, class V>
 __global__ __launch_bounds__(64) void prefix_waves_kernel(PrefixArgs a) {
@@ -744,19 +745,18 @@ static PrefixPlan prefix_plan(int64_t N, int64_t Hq, int64_t Hkv, int64_t P, int
   }
   p.n_wg_mixed = p.units ? (p.n_prefix_items + p.units - 1) / p.units + n_suffix : p.n_items;
   // More items than the mixed launch runs in one round: single waves (prefix_waves_kernel), up to 96 rows.  us, waves
-  // against the mixed launch (8 KV heads): N = 24, P = 8192 in pages, S <= 1000 30.3 against 33.4; N = 16, P = 16384,
-  // S = 1024 33.7 / 36.4; N = 6 of 8 rows a head, P = 8192 in NHD pages, S <= 500 25.1 / 31.1; N = 13, P = 7409, S = 34
+  // against the mixed launch (8 KV heads): N = 24, P = 8192 in pages, S <= 1000 30.3 against 33.4; N = 16, P = 16384, S
+  // = 1024 33.7 / 36.4; N = 6 of 8 rows a head, P = 8192 in NHD pages, S <= 500 25.1 / 31.1; N = 13, P = 7409, S = 34
   // 17.4 / 20.9.  At 128 rows four waves read every prefix tile and the rounds even out: N = 32, P = 4096, S = 256 22.3
-  // / 22.0; N = 32, P = 32768, S = 1000 69.5 / 63.0.  Grids of one round stay mixed: N = 8, P = 2048, S = 256 16.4 / 13.7.
-  // Up to 32 rows the gain is as large: 32 KV heads, N = 12, P = 2048, S = 32 16.4 / 24.1.  Over 2600 shapes of 2 to 96
-  // rows waves take 0.82 of the mixed launch's time in the mean, and more than 1.02 in 40 (at most 1.13: N = 32 of 2
-  // rows, 512 suffixes of 2048 after a prefix of 500).
-  // Full suffixes that take one round by themselves and are most of the work leave a second round little to do, and the
-  // merge launch is not won back: 16 KV heads of 2 rows, N = 16, P = 2048, S = 1024 29.7 / 27.4; 8 KV heads of 4, N = 24,
-  // P = 1000, S = 2048 39.1 / 36.3.  They stay mixed where the suffix tiles are at least 5 times the prefix's (10 times,
-  // past 32 rows); below that waves win: N = 16 of 2 rows, P = 8192, S = 1024 37.2 / 38.0; 8 KV heads of 1 row, N = 32,
-  // P = 8192, S = 1024 32.5 / 37.1.  Lengths below S leave the rounds uneven, and waves win again (N = 16 of 2 rows,
-  // P = 2048, S <= 1024 23.0 / 23.6).
+  // / 22.0; N = 32, P = 32768, S = 1000 69.5 / 63.0.  Grids of one round stay mixed: N = 8, P = 2048, S = 256 16.4 /
+  // 13.7. Up to 32 rows the gain is as large: 32 KV heads, N = 12, P = 2048, S = 32 16.4 / 24.1.  Over 2600 shapes of 2
+  // to 96 rows waves take 0.82 of the mixed launch's time in the mean, and more than 1.02 in 33 (at most 1.14: N = 32
+  // of 2 rows, 512 suffixes of 2048 after a prefix of 500). Full suffixes that take one round by themselves and are
+  // most of the work leave a second round little to do, and the merge launch is not won back: 16 KV heads of 2 rows, N
+  // = 16, P = 2048, S = 1024 29.7 / 27.4; 8 KV heads of 4, N = 24, P = 1000, S = 2048 39.1 / 36.3.  They stay mixed
+  // where the suffix tiles are at least 5 times the prefix's (10 times, past 32 rows); below that waves win: N = 16 of
+  // 2 rows, P = 8192, S = 1024 37.2 / 38.0; 8 KV heads of 1 row, N = 32, P = 8192, S = 1024 32.5 / 37.1.  Lengths below
+  // S leave the rounds uneven, and waves win again (N = 16 of 2 rows, P = 2048, S <= 1024 23.0 / 23.6).
   const int64_t suffix_tiles = n_suffix * (p.chunk_s / kTile), prefix_tiles = Hkv * ((P + kTile - 1) / kTile);
   const bool one_suffix_round = !ragged && S > 512 && n_suffix <= kDeviceCUs &&
                                 suffix_tiles >= (R <= 32 ? 5 : 10) * prefix_tiles * ((R + 31) / 32);
