@@ -604,7 +604,8 @@ template <class E>
 __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) {
   typedef part_t<E> PT;
   __shared__ float redm[4], sm[16], sl[16];
-  __shared__ __attribute__((aligned(16))) float so[16][128];   // rounded to PT, but for wide splits
+  __shared__ __attribute__((aligned(16))) float so_f[16 * 128];   // the splits' rows: fp32 if wide, else PT
+  PT* const so_h = reinterpret_cast<PT*>(so_f);
   const int tid = threadIdx.x, c = tid & 15, s = tid >> 4;
   const int R = a.kd * a.G;
   const int grel = blockIdx.x / R, row = blockIdx.x - grel * R;
@@ -686,11 +687,16 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
     for (int k = 0; k < 8; ++k) {
       acc[k] *= inv;
       asm("" : "+v"(acc[k]));                               // rounded to fp32 first, not fused with the conversion
-      if (!wide) acc[k] = (float)(PT)acc[k];
     }
+    auto put = [&](auto* so) {
 #pragma unroll
-    for (int k = 0; k < 8; k += 4)
-      store_part4(&so[s][8 * c + k], floatx4{acc[k], acc[k + 1], acc[k + 2], acc[k + 3]});
+      for (int k = 0; k < 8; k += 4)
+        store_part4(so + s * 128 + 8 * c + k, floatx4{acc[k], acc[k + 1], acc[k + 2], acc[k + 3]});
+    };
+    if (wide)
+      put(so_f);
+    else
+      put(so_h);
   };
   float M = kNegInf;
   if (nsplit > 16) {                                        // the largest m before the first weight
@@ -713,16 +719,22 @@ __global__ __launch_bounds__(256) void key_units_combine_kernel(KeySplitArgs a) 
         }
         M = (M == kNegInf) ? 0.f : M;
       }
-      for (int j = 0; j < ns; ++j) {
-        const float w = part_weight(float2{sm[j], sl[j]}, M);
-        den += w;
-        num += w * so[j][tid];
-      }
+      auto add = [&](const auto* so) {
+        for (int j = 0; j < ns; ++j) {
+          const float w = part_weight(float2{sm[j], sl[j]}, M);
+          den += w;
+          num += w * (float)so[j * 128 + tid];
+        }
+      };
+      if (wide)
+        add(so_f);
+      else
+        add(so_h);
     }
   }
   if (tid >= 128) return;
   if (nsplit == 1) {                                        // the split is the result, as key_split_kernel writes it
-    num = sl[0] == 0.f ? __builtin_nanf("") : so[0][tid];
+    num = sl[0] == 0.f ? __builtin_nanf("") : wide ? so_f[tid] : (float)so_h[tid];
     den = 1.f;
   }
   const int di = row / a.G, gg = row - di * a.G;
